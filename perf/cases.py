@@ -94,6 +94,8 @@ def draw(rng):
         if joint:
             case["H"] = rng.choice([256, 320, 384, 512, 640])
             case["dropout"] = rng.choice([0.0, 0.2])
+        if case["steps"].startswith("1") and op.endswith("tdt") and 2 * case["U"] > case["T"]:
+            continue  # no duration 0: a frame a label, and some utterances would have no alignment
         need = work(case)
         if (case["B"] * case["T"] * case["U"] <= cells_limit and need["bytes"] <= max(w["bytes"] for w in largest)
                 and (not joint or need["flops"] <= max(w["flops"] for w in largest))):  # fmt: skip
@@ -124,7 +126,7 @@ def _lengths(case):
     return out
 
 
-def prepare(case, seed):
+def _inputs(case, seed):
     device = torch.device("cuda")
     gen = torch.Generator(device=device).manual_seed(seed)
     host = torch.Generator().manual_seed(seed)
@@ -155,7 +157,14 @@ def prepare(case, seed):
     for b in range(B):
         acts[b] = torch.randn(T, U, _row(case), generator=gen, device=device) * case["std"]
     state["acts"] = acts.requires_grad_(case["train"])
-    options = dict(fastemit_lambda=case["fastemit"], clamp=case["clamp"])
+    if case["op"] == "logprobs":  # the graph loss hands back a gradient of the scores
+        state["grad_scores"] = [-torch.rand(B, T, U, generator=gen, device=device) for _ in range(2)]
+    return state
+
+
+def prepare(case, seed):
+    state = _inputs(case, seed)
+    V, options = case["V"], dict(fastemit_lambda=case["fastemit"], clamp=case["clamp"])
     if case["op"] == "rnnt":
         state["loss"] = RNNTLossNumba(blank=V - 1, reduction="none", **options)
     elif case["op"] == "wrapper":
@@ -165,8 +174,6 @@ def prepare(case, seed):
     elif case["op"] == "multiblank":
         state["loss"] = MultiblankRNNTLossNumba(blank=V - 1, big_blank_durations=_steps(case), reduction="none",
                                                 sigma=case["sigma"], **options)  # fmt: skip
-    else:  # logprobs: the graph loss hands back a gradient of the scores
-        state["grad_scores"] = [-torch.rand(B, T, U, generator=gen, device=device) for _ in range(2)]
     return state
 
 
@@ -236,3 +243,145 @@ def tolerance(case):
     if case["dtype"] == "float16":
         return {"rel": 9e-4, "max": 2e-3}
     return {"rel": 6e-6, "max": 1.6e-4}
+
+
+def _arcs(case):
+    """(frames, labels, token, place of its duration or None) of every arc out of a cell; a big blank's token is its place."""
+    if case["op"].endswith("tdt"):
+        steps = list(enumerate(_steps(case)))
+        return [(d, 0, "blank", i) for i, d in steps if d > 0] + [(d, 1, "label", i) for i, d in steps]
+    arcs = [(1, 0, "blank", None), (0, 1, "label", None)]
+    if case["op"].endswith("multiblank"):
+        arcs += [(d, 0, i, None) for i, d in enumerate(_steps(case))]
+    return arcs
+
+
+def _lattice(case, lengths, tokens, durations):
+    """Log-likelihood of each utterance and the posterior of every arc, from log-probs [B, T, U] in 64 bits: the forward
+    and the backward recursion over anti-diagonals n = t + u, all utterances at once."""
+    B, T, U, device = case["B"], case["T"], case["U"], tokens["blank"].device
+    frames = torch.tensor([t for t, _ in lengths], device=device)[:, None, None]
+    labels = torch.tensor([u for _, u in lengths], device=device)[:, None, None]
+    t, u = torch.arange(T, device=device)[:, None], torch.arange(U, device=device)
+    N = T + U - 1
+    n = torch.arange(N, device=device)[:, None]
+    at = (n - u).clamp(0, T - 1)  # the frame of diagonal n, column u
+    on = (n >= u) & (n - u < T)
+
+    def skew(x, fill=-math.inf):
+        return x[:, at, u].masked_fill(~on, fill).transpose(0, 1).contiguous()  # [N, B, U]
+
+    inside, ends = [], []
+    for dt, du, token, place in _arcs(case):
+        score = tokens[token] - case["sigma"] + (durations[..., place] if place is not None else 0.0)
+        valid = (t < frames) & (u <= labels)
+        inside.append(skew(score.masked_fill(~(valid & (t + dt < frames) & (u + du <= labels)), -math.inf)))
+        ends.append(skew(score.masked_fill(~(valid & (t + dt == frames) & (u == labels)), -math.inf)) if du == 0 else None)
+    finish = torch.logsumexp(torch.stack([e for e in ends if e is not None]), 0)
+    shifts = [(dt, du) for dt, du, _, _ in _arcs(case)]
+    most = max(dt + du for dt, du in shifts)
+    alpha = torch.full((N + most, B, U), -math.inf, dtype=torch.float64, device=device)  # row n + most: diagonal n
+    beta = torch.full((N + most, B, U + 1), -math.inf, dtype=torch.float64, device=device)
+    alpha[most, :, 0] = 0.0
+    for k in range(1, N):
+        terms = torch.full((len(shifts), B, U), -math.inf, dtype=torch.float64, device=device)
+        for i, (dt, du) in enumerate(shifts):
+            if k >= dt + du:
+                terms[i, :, du:] = (alpha[most + k - dt - du] + inside[i][k - dt - du])[:, : U - du]
+        alpha[most + k] = torch.logsumexp(terms, 0)
+    for k in reversed(range(N)):
+        terms = [finish[k]] + [beta[k + dt + du][:, du : U + du] + inside[i][k] for i, (dt, du) in enumerate(shifts)]
+        beta[k, :, :U] = torch.logsumexp(torch.stack(terms), 0)
+    ll = beta[0, :, 0]
+    posteriors = []
+    for i, (dt, du) in enumerate(shifts):
+        through = torch.exp(alpha[most:] + inside[i] + beta[dt + du : dt + du + N, :, du : U + du] - ll[:, None])
+        if ends[i] is not None:
+            through += torch.exp(alpha[most:] + ends[i] - ll[:, None])
+        posteriors.append(through[t + u, :, u].permute(2, 0, 1))  # back to [B, T, U]
+    return ll, posteriors
+
+
+def exact(case, seed):
+    """What `run` returns, in 64 bits: log-softmax, the lattice's arc posteriors and the Jacobian of the softmax, by
+    definition.  None with dropout, whose mask only the joint's kernels know."""
+    if case["dropout"]:
+        return None
+    s = _inputs(case, seed)
+    B, T, U, V = case["B"], case["T"], case["U"], case["V"]
+    steps = _steps(case)
+    is_tdt = case["op"].endswith("tdt")
+    joint = case["op"].startswith("joint")
+    lengths = list(zip(s["act_lens"].tolist(), s["label_lens"].tolist()))
+    ids = torch.cat([s["labels"], s["labels"].new_zeros(B, 1)], 1)
+
+    def hidden(b):
+        return torch.relu(s["f"][b].detach().double()[:, None] + s["g"][b].detach().double())
+
+    def logits(b):
+        if joint:
+            return hidden(b) @ s["weight"].detach().double().T + s["bias"].detach().double()
+        return s["acts"][b].detach().double()
+
+    which = {"blank": V - 1, **{i: V - 2 - i for i in range(len(steps) if case["op"].endswith("multiblank") else 0)}}
+    picked, of_durations = {k: [] for k in ("label", *which)}, []
+    for b in range(B):
+        x = logits(b)
+        norm = torch.logsumexp(x[..., :V], -1)
+        picked["label"].append(x.gather(-1, ids[b].expand(T, U)[..., None])[..., 0] - norm)
+        for k, v in which.items():
+            picked[k].append(x[..., v] - norm)
+        of_durations.append(torch.log_softmax(x[..., V:], -1) if is_tdt else None)
+    tokens = {k: torch.stack(v) for k, v in picked.items()}
+    durations = torch.stack(of_durations) if is_tdt else None
+
+    if case["op"] == "logprobs":
+        t, u = torch.arange(T, device=ids.device)[:, None], torch.arange(U, device=ids.device)
+        cell = (t < s["act_lens"][:, None, None]) & (u <= s["label_lens"][:, None, None])
+        target = cell & (u < s["label_lens"][:, None, None])
+        scores = (tokens["label"].masked_fill(~target, 0.0), tokens["blank"].masked_fill(~cell, 0.0))
+        flow = {"label": -s["grad_scores"][0].double() * target, "blank": -s["grad_scores"][1].double() * cell}
+        costs, of_places = None, []
+    else:
+        ll, posteriors = _lattice(case, lengths, tokens, durations)
+        costs = -ll * (1.0 + case["fastemit"])
+        flow = {k: torch.zeros(B, T, U, dtype=torch.float64, device=ids.device) for k in tokens}
+        of_places = [torch.zeros_like(flow["blank"]) for _ in steps] if is_tdt else []
+        for (_, _, token, place), p in zip(_arcs(case), posteriors):
+            flow[token] += p * (1.0 + case["fastemit"]) if token == "label" else p
+            if place is not None:
+                of_places[place] += p
+    scale = 1.0
+    if case["op"] == "wrapper":
+        costs, scale = costs.mean(), 1.0 / B
+    if not case["train"]:
+        return costs
+
+    total = sum(flow.values())
+    if joint:
+        grads = [torch.zeros(x.shape, dtype=torch.float64, device=x.device) for x in (s["f"], s["g"], s["weight"], s["bias"])]
+    else:
+        grads = torch.zeros(s["acts"].shape, dtype=torch.float64, device=ids.device)
+    for b in range(B):
+        x = logits(b)
+        x[..., :V] = torch.softmax(x[..., :V], -1) * total[b][..., None]
+        x.scatter_add_(-1, ids[b].expand(T, U)[..., None], -flow["label"][b][..., None])
+        for k, v in which.items():
+            x[..., v] -= flow[k][b]
+        if is_tdt:
+            place = torch.stack([p[b] for p in of_places], -1)
+            x[..., V:] = torch.exp(durations[b]) * place.sum(-1, keepdim=True) - place
+        if case["clamp"] > 0.0:
+            x.clamp_(-case["clamp"], case["clamp"])
+        if not joint:
+            grads[b] = x * scale
+            continue
+        h, rows = hidden(b), x.reshape(T * U, -1)
+        through = (x @ s["weight"].detach().double()) * (h > 0)
+        grads[0][b] = through.sum(1)
+        grads[1][b] = through.sum(0)
+        grads[2] += rows.T @ h.reshape(T * U, -1)
+        grads[3] += rows.sum(0)
+    if joint:
+        return (costs, *grads)
+    return (*scores, grads) if case["op"] == "logprobs" else (costs, grads)
