@@ -260,4 +260,62 @@ inline long long plan_blocks(const PlanShape& s, const BlockPlan& p) { return (l
 inline int row_chunks(const PlanShape& s, int rpw) { return (s.U + kRowWaves * rpw - 1) / (kRowWaves * rpw); }
 inline long long row_blocks(const PlanShape& s, int rpw) { return (long long)row_chunks(s, rpw) * s.B * s.T; }
 
+// Short rows (at most 64 whole vectors): both passes take tiles of 1 << log_rows consecutive rows of one frame
+// (mi_tile.inc), as many as make up to 16 KB -- four 16-byte vectors a thread -- and no more than a frame needs.  Eight
+// rows always fit (they are at most 9 KB).  Longer rows keep the kernels that give a row whole waves: from 65 vectors
+// on every lane has work there (measured figures: mi_tile.inc).
+constexpr int kTileBytes = 16 * 1024 - 16;
+constexpr int kTileMaxRows = 128;
+struct RowTile {
+  int log_rows;  // 0: not a short row
+  int rows() const { return 1 << log_rows; }
+};
+inline RowTile row_tile(const PlanShape& s) {
+  if (!MI_USE_ROWS || s.whole_vectors() > 64) return RowTile{0};
+  const long long row_bytes = (long long)(s.V + s.D) * (16 / s.vec());
+  int log_rows = 3;
+  while ((2 << log_rows) <= kTileMaxRows && (row_bytes << (log_rows + 1)) <= kTileBytes && (1 << log_rows) < s.U) ++log_rows;
+  return RowTile{log_rows};
+}
+inline int tile_chunks(const PlanShape& s, const RowTile& t) { return (s.U + t.rows() - 1) >> t.log_rows; }
+inline long long tile_blocks(const PlanShape& s, const RowTile& t) { return (long long)tile_chunks(s, t) * s.B * s.T; }
+// Pass 1 over them: as many cells, but 16 (or a power of two that holds U) rows of each of several frames.
+constexpr int kTileMaxFrames = 16;
+struct DenomTile {
+  int log_rows, log_frames;  // log_rows + log_frames: 3 ... 7
+  int frame_groups;          // groups of frames per utterance
+  int pitch;                 // 16-byte vectors that hold a frame's rows wherever they start
+  FastDiv div_pitch;
+};
+inline DenomTile denom_tile(const PlanShape& s) {
+  const long long row_bytes = (long long)(s.V + s.D) * (16 / s.vec());
+  int log_cells = 3;
+  while ((2 << log_cells) <= kTileMaxRows && (row_bytes << (log_cells + 1)) <= kTileBytes) ++log_cells;
+  DenomTile d;
+  d.log_rows = 0;
+  while (d.log_rows < 4 && d.log_rows < log_cells && (1 << d.log_rows) < s.U) ++d.log_rows;
+  d.log_frames = log_cells - d.log_rows;
+  if ((1 << d.log_frames) > kTileMaxFrames) d.log_frames = 4;
+  if (d.log_rows + d.log_frames < 3) d.log_frames = 3 - d.log_rows;
+  d.frame_groups = (s.T + (1 << d.log_frames) - 1) >> d.log_frames;
+  d.pitch = (int)(((row_bytes << d.log_rows) + 15) / 16) + 1;
+  d.div_pitch = make_fastdiv((unsigned)d.pitch);
+  return d;
+}
+inline int denom_tile_chunks(const PlanShape& s, const DenomTile& d) { return (s.U + (1 << d.log_rows) - 1) >> d.log_rows; }
+inline long long denom_tile_blocks(const PlanShape& s, const DenomTile& d) {
+  return (long long)denom_tile_chunks(s, d) * s.B * d.frame_groups;
+}
+// Consecutive tiles per XCD and turn: 64 (a tile's cells read the lattice diagonals of the neighbouring frames', which
+// should find them in the same level-2 cache), fewer where the grid would not give every XCD four turns.
+inline int tile_log_span(long long blocks) {
+  int log_span = 6;
+  while (log_span > 0 && (32LL << log_span) > blocks) --log_span;
+  return log_span;
+}
+inline unsigned tile_grid(long long blocks) {
+  const long long turn = 8LL << tile_log_span(blocks);
+  return (unsigned)((blocks + turn - 1) / turn * turn);
+}
+
 #endif  // MI_PLAN_H_

@@ -1,7 +1,7 @@
 // MI355X (gfx950, wave64) transducer-loss kernels and their C ABI (include/mi_transducer.h).
 //
 // Pipeline of a forward + backward call (one stream, no host synchronisation, nothing allocated):
-//   pass 1   denom_rows_kernel | denom_block_kernel | denom_gather_kernel      (mi_streaming.inc)
+//   pass 1   denom_tile_kernel (mi_tile.inc) | denom_rows_kernel | denom_block_kernel | denom_gather_kernel (mi_streaming.inc)
 //            streams the valid rows of acts once (16-byte aligned loads, log-sum-exp per row) and leaves per
 //            cell the denominator and, as one record of consecutive floats, the blank / label (/ duration /
 //            big-blank) log-probabilities, the records in a SKEWED layout [b][t+u][u][record], so that an
@@ -10,9 +10,10 @@
 //            | multiblank_lattice_kernel | multiblank_lattice_pull_kernel        (mi_multiblank.inc)
 //            alpha and beta over the anti-diagonals, accumulated in fp64 (only the log1p(exp(.)) term in fp32);
 //            the alpha side writes costs.
-//   cells    tdt_cell_kernel | multiblank_cell_kernel (RNNT: none, the gradient pass derives them itself)
+//   cells    tdt_cell_kernel | multiblank_cell_kernel | rnnt_cell_kernel (RNNT rows of more than 64 vectors: none, the gradient
+//            pass derives them itself)
 //            one thread per lattice cell: the few numbers a gradient row needs, grad_scale folded in.
-//   pass 2   grad_rows_kernel | grad_block_kernel | grad_stream_kernel          (mi_streaming.inc)
+//   pass 2   grad_tile_kernel (mi_tile.inc) | grad_block_kernel | grad_stream_kernel   (mi_streaming.inc)
 //            streams acts a second time and writes every gradient element once, zeros for padded cells included.
 // The compact log-prob op (mi_logprobs.inc) reuses pass 1 and pass 2; the fused joint + loss (mi_joint.inc) replaces
 // pass 1 and the producer of the logits by an MFMA kernel.  Host-side checks and launchers: mi_host.inc.
@@ -54,6 +55,7 @@ namespace {
 #include "mi_logprobs.inc"
 #include "mi_multiblank.inc"
 #include "mi_streaming.inc"
+#include "mi_tile.inc"
 #include "mi_host.inc"
 
 }  // namespace
@@ -534,6 +536,8 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   char denom[96], lattice[96], cells[48], grad[112];
   const BlockPlan dp = denom_block_plan(c);
   if (dp.RT) snprintf(denom, sizeof denom, "denom_block_kernel<%s, RT=%d, NVT=%d>", dt, dp.RT, dp.NVT);
+  // R=1: short rows, the tile kernels of mi_tile.inc (RPW: the vectors of a tile a thread moves)
+  else if (row_tile(c).log_rows) snprintf(denom, sizeof denom, "denom_rows_kernel<%s, R=1, RPW=%d>", dt, kTileRounds);
   else if (denom_rows_R(c)) snprintf(denom, sizeof denom, "denom_rows_kernel<%s, R=%d, RPW=%d>", dt, denom_rows_R(c), denom_rows_per_wave(denom_rows_R(c)));
   else snprintf(denom, sizeof denom, "denom_gather_kernel<%s>", dt);
   const bool tdt = D > 0 && !use_plain_rnnt;
@@ -556,7 +560,7 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   const bool fused = !tdt && !mb && rnnt_rows_fused(c, nullptr);
   snprintf(cells, sizeof cells, "%s", fused ? "-" : (mb ? "multiblank_cell_kernel" : (tdt ? "tdt_cell_kernel" : "rnnt_cell_kernel")));
   if (gp.RT) snprintf(grad, sizeof grad, "grad_block_kernel<%s, RT=%d, NVT=%d, %s>", dt, gp.RT, gp.NVT, fused ? "fused" : "coef");
-  else if (rows_R(c)) snprintf(grad, sizeof grad, "grad_rows_kernel<%s, R=%d, %s>", dt, rows_R(c), fused ? "fused" : "coef");
+  else if (row_tile(c).log_rows) snprintf(grad, sizeof grad, "grad_rows_kernel<%s, R=1, coef>", dt);
   else snprintf(grad, sizeof grad, "grad_stream_kernel<%s>", dt);
   const int n = snprintf(out, out_bytes, "denominators=%s; lattice=%s; cells=%s; gradient=%s%s", denom, lattice, cells,
                          grad, (mb && !gp.RT) ? " + multiblank_fixup_kernel" : "");
