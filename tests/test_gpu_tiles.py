@@ -65,3 +65,17 @@ def test_multiblank(U, V):
     loss = MultiblankRNNTLossNumba(blank=V - 1, big_blank_durations=[2, 4], reduction="none", sigma=0.05)
     want = oracle.multiblank_loss(x.double().numpy(), *rest, V - 1, [2, 4], 0.05)
     _check(_run(loss, x, *rest), want, F32)
+
+
+@pytest.mark.parametrize("U", [129, 193, 257, 500, 1000])
+def test_wide_label_axis(U):
+    """The RNNT recursion in workgroups of 4, 8 and 16 waves: utterances that end beside a wave's edge and fewer
+    diagonals than a batch."""
+    rng = np.random.RandomState(U)
+    B, T, V = 4, 5, 4
+    x = torch.tensor(rng.randn(B, T, U, V))
+    labels = rng.randint(0, V - 1, size=(B, U - 1))
+    act_lens, label_lens = np.array([T, 1, 3, 4]), np.array([U - 1, 2, 63, 128])
+    loss = RNNTLossNumba(blank=V - 1, reduction="none")
+    want = oracle.rnnt_loss(x.float().double().numpy(), labels, act_lens, label_lens, V - 1)
+    _check(_run(loss, x.float(), labels, act_lens, label_lens), want, F32)
