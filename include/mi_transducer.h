@@ -388,6 +388,11 @@ int mi_transducer_export_lattice(const void* workspace, size_t workspace_bytes, 
 int mi_transducer_length_maxima(const int64_t* act_lens, const int64_t* label_lens, int B, int64_t* out,
                                 void* stream);
 
+/* With `out` in pinned host memory the kernel writes the two words straight to the host.  This call returns once both
+ * are there: the caller sets them to INT64_MIN before it enqueues the kernel on `stream` (not one that is being
+ * captured).  No event, and nothing that was enqueued behind the kernel is waited for. */
+int mi_transducer_wait_lengths(const int64_t* words, void* stream);
+
 /* ---- diagnostics ------------------------------------------------------------------------
  * Everything from here to the end of this header (mi_transducer_profile_*, mi_transducer_describe_plan,
  * mi_transducer_copy_probe, mi_transducer_prefill_record) binds NO interface of the reference: these are aids for

@@ -24,6 +24,7 @@
 
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <sched.h>
 #include <stdio.h>
 #include <stdint.h>
 #include <stdlib.h>
@@ -68,7 +69,7 @@ namespace {
 // ----------------------------------------------------------------------------------------
 extern "C" {
 
-int mi_transducer_abi_version(void) { return 20; }
+int mi_transducer_abi_version(void) { return 21; }
 
 int mi_transducer_workspace_bytes(int B, int T, int U, int D, size_t* out_bytes) {
   Layout L;
@@ -416,6 +417,22 @@ int mi_transducer_length_maxima(const int64_t* act_lens, const int64_t* label_le
   if (!act_lens || !label_lens || !out || B <= 0) return MI_TRANSDUCER_INVALID_VALUE;
   hipLaunchKernelGGL(length_maxima_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, act_lens, label_lens, B, out);
   return launch_status();
+}
+
+int mi_transducer_wait_lengths(const int64_t* words, void* stream) {
+  if (!words) return MI_TRANSDUCER_INVALID_VALUE;
+  const volatile int64_t* w = words;
+  for (unsigned long long look = 1;; ++look) {
+    if (w[0] != INT64_MIN && w[1] != INT64_MIN) return MI_TRANSDUCER_SUCCESS;
+    if (look % 64 == 0) sched_yield();
+    // now and then, has the stream finished or failed?  (its answer is final: the words hold whatever was written)
+    if (look % 16384 == 0) {
+      const hipError_t state = hipStreamQuery((hipStream_t)stream);
+      if (state == hipSuccess) return MI_TRANSDUCER_SUCCESS;
+      if (state != hipErrorNotReady) return MI_TRANSDUCER_LAUNCH_FAILURE;
+    }
+    __builtin_ia32_pause();
+  }
 }
 
 int mi_transducer_denominators(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,

@@ -16,7 +16,7 @@ import torch
 
 from speech_amd import _native
 from speech_amd.rnnt_loss.rnnt_pytorch import grads_like
-from speech_amd.rnnt_loss.rnnt import _dtype_code, _labels_ptr, _ptr, _require_gpu, _stream, new_workspace
+from speech_amd.rnnt_loss.rnnt import _dtype_code, _labels_ptr, _on, _ptr, _require_gpu, _stream, new_workspace
 
 __all__ = ["RnntLogProbs", "rnnt_logprobs", "rnnt_logprobs_triton"]
 
@@ -46,7 +46,7 @@ class RnntLogProbs(torch.autograd.Function):
         target_scores = torch.empty(B, T, U, dtype=torch.float32, device=device)
         blank_scores = torch.empty_like(target_scores)
         workspace = new_workspace(logits)
-        with torch.cuda.device(device):
+        with _on(device):
             status = _native.lib().mi_rnnt_logprobs_forward(
                 _ptr(logits), _dtype_code(logits), _labels_ptr(targets), _ptr(source_lengths), _ptr(target_lengths),
                 _ptr(target_scores), _ptr(blank_scores), B, T, U, V, int(blank_id), _ptr(workspace),
@@ -69,7 +69,7 @@ class RnntLogProbs(torch.autograd.Function):
         grad_target_scores = grad_target_scores.to(torch.float32).contiguous()
         grad_blank_scores = grad_blank_scores.to(torch.float32).contiguous()
         grad_logits = grads_like(logits)  # every element is written, padded cells as zeros
-        with torch.cuda.device(device):
+        with _on(device):
             status = _native.lib().mi_rnnt_logprobs_backward(
                 _ptr(logits), _dtype_code(logits), _labels_ptr(targets), _ptr(source_lengths), _ptr(target_lengths),
                 _ptr(grad_target_scores), _ptr(grad_blank_scores), _ptr(grad_logits), have_state, B, T, U, V,

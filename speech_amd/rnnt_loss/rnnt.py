@@ -19,6 +19,7 @@ Differences a caller can see:
   * these functions run on the GPU only (the module-level RNNT loss has a CPU path of its own).
 """
 
+import contextlib
 import ctypes
 import random
 
@@ -51,6 +52,14 @@ def _ptr(t):
 
 def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on(device):
+    """torch.cuda.device(device), without its cost where that is the current device already."""
+    return _NO_SWITCH if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _labels_ptr(labels):
@@ -88,12 +97,23 @@ def length_maxima(act_lens, label_lens, out=None):
         out = torch.empty(2, dtype=torch.int64, device=act_lens.device)
     elif out.dtype != torch.int64 or out.numel() != 2 or not (out.is_cuda or out.is_pinned()):
         raise ValueError("length_maxima: out must be an int64[2] device or pinned host tensor")
-    with torch.cuda.device(act_lens.device):
+    with _on(act_lens.device):
         status = _native.lib().mi_transducer_length_maxima(
             _ptr(act_lens), _ptr(label_lens), act_lens.shape[0], _ptr(out), _stream(act_lens.device)
         )
     _native.check_status(status, "length_maxima")
     return out
+
+
+# what the caller of wait_lengths leaves in the two words before it enqueues length_maxima(out=words)
+LENGTHS_PENDING = -(2**63)
+
+
+def wait_lengths(words, stream):
+    """Return once the kernel of length_maxima(..., out=words), enqueued on `stream`, has written both words (a pinned
+    host tensor that held LENGTHS_PENDING before)."""
+    status = _native.lib().mi_transducer_wait_lengths(_ptr(words), ctypes.c_void_p(stream.cuda_stream))
+    _native.check_status(status, "length check")
 
 
 def zero_padding(grads, act_lens, label_lens):
@@ -148,7 +168,7 @@ def rnnt_forward(acts, labels, act_lens, label_lens, costs, blank, fastemit_lamb
     _require_gpu(acts, "rnnt_forward")
     B, T, U, V = acts.shape
     _check_prefill(acts, prefill_grads)
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_rnnt_forward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, V, int(blank), float(fastemit_lambda), int(bool(with_betas)), _ptr(prefill_grads),
@@ -166,7 +186,7 @@ def rnnt_backward(
     and the current stream waits for it (1), or the forward call was given grads as prefill_grads (2)."""
     _require_gpu(acts, "rnnt_backward")
     B, T, U, V = acts.shape
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_rnnt_backward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(grads),
             _ptr(grad_scale), int(grad_scale_stride), float(grad_mul), int(padding_zeroed), B, T, U, V, int(blank),
@@ -185,7 +205,7 @@ def tdt_forward(
     _check_prefill(acts, prefill_grads)
     D = len(durations)
     keep, dur_ptr = _durations_array(durations)
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_tdt_forward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, VD - D, D, dur_ptr, int(blank), float(fastemit_lambda), float(sigma), int(bool(use_plain_rnnt)),
@@ -203,7 +223,7 @@ def tdt_backward(
     B, T, U, VD = acts.shape
     D = len(durations)
     keep, dur_ptr = _durations_array(durations)
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_tdt_backward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(grads),
             _ptr(grad_scale), int(grad_scale_stride), float(grad_mul), int(padding_zeroed), B, T, U, VD - D, D,
@@ -223,7 +243,7 @@ def multiblank_forward(
     B, T, U, V = acts.shape
     _check_prefill(acts, prefill_grads)
     keep, dur_ptr = _durations_array(big_blank_durations)
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_multiblank_forward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, V, len(big_blank_durations), dur_ptr, int(blank), float(fastemit_lambda), float(sigma),
@@ -240,7 +260,7 @@ def multiblank_backward(
     _require_gpu(acts, "multiblank_backward")
     B, T, U, V = acts.shape
     keep, dur_ptr = _durations_array(big_blank_durations)
-    with torch.cuda.device(acts.device):
+    with _on(acts.device):
         status = _native.lib().mi_multiblank_backward(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(grads),
             _ptr(grad_scale), int(grad_scale_stride), float(grad_mul), int(padding_zeroed), B, T, U, V,

@@ -21,11 +21,12 @@ What is done differently underneath:
     `acts`, as the reference does (which computes the gradient there): the lattice launch
     zero-fills its padded cells while it runs.  That tensor is held until backward runs or
     the graph is dropped; MI_TRANSDUCER_PREFILL=0 in the environment restores the small footprint.
-  * the shape-vs-lengths check reads both maxima back with one small copy that
-    overlaps the forward kernels instead of two blocking torch.max calls.
+  * the shape-vs-lengths check has one small kernel write both maxima into host memory and
+    looks at them once the forward kernels are enqueued, instead of two blocking torch.max calls.
 """
 
 import contextlib
+import ctypes
 import os
 import random
 import threading
@@ -59,15 +60,20 @@ def _prefill_wanted(acts):
     return acts.numel() * acts.element_size() >= _PREFILL_MIN_BYTES
 
 
-_aux_streams = {}
+class _LengthWords(threading.local):
+    """Two pinned words per thread and the tensor that owns them: where the length check of a call finds the maxima.  A
+    call is done with them before it returns, so one pair serves all calls of a thread, on whatever stream or device."""
+
+    tensor = words = None
+
+    def get(self):
+        if self.tensor is None:
+            self.tensor = torch.empty(2, dtype=torch.int64, pin_memory=True)
+            self.words = (ctypes.c_int64 * 2).from_address(self.tensor.data_ptr())
+        return self.tensor, self.words
 
 
-def _aux_stream(device):
-    stream = _aux_streams.get(device.index)
-    if stream is None:
-        stream = torch.cuda.Stream(device=device)  # default priority
-        _aux_streams[device.index] = stream
-    return stream
+_length_words = _LengthWords()
 
 
 def grads_like(acts):
@@ -152,35 +158,32 @@ class _PendingLengthCheck:
         self.padded_T = _caller_mode.padded_time_axis
         self.key = (lengths._version, label_lengths._version, self.T, self.U, self.padded_T)
         self.tensors = (lengths, label_lengths)
-        self.event = self.host = None
+        self.host = self.stream = None
         seen = _validated.entry
         if (not _STRICT_LENGTH_CHECK and seen is not None and seen[0]() is lengths and seen[1]() is label_lengths
                 and seen[2] == self.key):
             return  # these very tensors, unmodified, passed against this shape
         if lengths.is_cuda:
-            # One small kernel on the auxiliary stream, ordered after whatever produced the lengths
-            # on the current stream, writes the two maxima into pinned host memory: it runs beside
-            # the first kernel of the loss instead of in front of it.
-            main = torch.cuda.current_stream(lengths.device)
-            aux = _aux_stream(lengths.device)
-            aux.wait_stream(main)
-            self.host = torch.empty(2, dtype=torch.int64, pin_memory=True)
-            with torch.cuda.stream(aux):
-                rnnt.length_maxima(lengths, label_lengths, out=self.host)
-                self.event = torch.cuda.Event()
-                self.event.record(aux)
-            lengths.record_stream(aux)
-            label_lengths.record_stream(aux)
+            # One small kernel in front of the first kernel of the loss, on the same stream, writes the two maxima into
+            # pinned host memory; finish() looks at the words until they are there.  (On a stream of its own, behind
+            # an event, the kernel overlaps pass 1, but the event leaves a gap in front of pass 1 that is longer than
+            # the kernel, and stream, events and record_stream cost the host 40 to 60 us a call.  Step at B=4, T=50,
+            # U=21, V=129 233 -> 166 us, forward alone at B=8, T=187, U=46, V=1025 85 -> 47 us.)
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("the shape check of new length tensors reads the lengths back: it cannot be captured")
+            self.host, words = _length_words.get()
+            words[0] = words[1] = rnnt.LENGTHS_PENDING
+            rnnt.length_maxima(lengths, label_lengths, out=self.host)
+            self.stream = torch.cuda.current_stream(lengths.device)
         else:
             self.host = torch.stack([torch.max(lengths), torch.max(label_lengths)])
 
     def drain(self):
-        """Wait for the kernel that writes into the pinned buffer, so that the buffer is not handed back to the host
-        allocator (and on to some other user) while that write is still queued.  For the error paths that drop
-        this object without finish()."""
-        if self.event is not None:
-            self.event.synchronize()
-            self.event = None
+        """Wait for the kernel that writes into the pinned words, so that the thread's next call does not find a late
+        write of this one there.  For the error paths that drop this object without finish()."""
+        if self.stream is not None:
+            rnnt.wait_lengths(self.host, self.stream)
+            self.stream = None
 
     def finish(self):
         if self.host is None:
