@@ -261,10 +261,11 @@ inline int row_chunks(const PlanShape& s, int rpw) { return (s.U + kRowWaves * r
 inline long long row_blocks(const PlanShape& s, int rpw) { return (long long)row_chunks(s, rpw) * s.B * s.T; }
 
 // Short rows (at most 64 whole vectors): both passes take tiles of 1 << log_rows consecutive rows of one frame
-// (mi_tile.inc), as many as make up to 16 KB -- four 16-byte vectors a thread -- and no more than a frame needs.  Eight
+// (mi_tile.inc), as many as make up to 17 KB -- four 16-byte vectors a thread and a few more, so that the usual vocabulary
+// sizes, a power of two and a blank (and durations), do not fall to half a tile -- and no more than a frame needs.  Eight
 // rows always fit (they are at most 9 KB).  Longer rows keep the kernels that give a row whole waves: from 65 vectors
 // on every lane has work there (measured figures: mi_tile.inc).
-constexpr int kTileBytes = 16 * 1024 - 16;
+constexpr int kTileBytes = 17 * 1024 - 16;
 constexpr int kTileMaxRows = 128;
 struct RowTile {
   int log_rows;  // 0: not a short row
