@@ -12,7 +12,7 @@ to the loss (:1573-1578); autograd then keeps that tensor and a gradient of the 
   backward  two kernels form the gradient of the logits from the saved ones on the fly and multiply it, on the
             matrix cores, with the weights (d hidden) and with the saved activations (d weight, d bias; partial sums
             per slice of the rows, added up here); a reduction kernel sums d hidden, in one pass, over u into d f
-            and over t into d g (d g as one partial sum per run of 32 frames, added up here).  No library GEMM, no
+            and over t into d g (d g as one partial sum per run of frames, added up here).  No library GEMM, no
             host wait.
 
 `joint_rnnt_loss` is differentiable in f, g, weight and bias; `joint_rnnt_forward` is the no-grad form.
@@ -291,9 +291,13 @@ class JointRNNTLoss(torch.autograd.Function):
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
             want_f, want_g = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
             d_f32 = torch.empty(B, T, H, dtype=torch.float32, device=device) if want_f else None
-            # both wanted (the usual case): one pass over d_hidden forms d f and, per run of 32 frames, a share of d g
-            # (runs of a fixed length: the sums then do not depend on how a batch is split into sub-batches)
-            chunks = (T + 31) // 32 if (want_f and want_g and U <= 256) else 0
+            # both wanted (the usual case): one pass over d_hidden forms d f and, per run of frames, a share of d g (runs
+            # of a length that U alone decides: the sums then do not depend on how a batch is split into sub-batches).
+            # A workgroup walks its run frame by frame, a barrier each; where a frame is short (U <= 64) its latency is
+            # the bound and runs of 16 frames are faster than runs of 32: B=4, T=190, U=49 48 -> 27 us, B=8, T=250, U=60
+            # 52 -> 49 us.  Longer frames keep 32, and half the partial sums.
+            run = 16 if U <= 64 else 32
+            chunks = (T + run - 1) // run if (want_f and want_g and U <= 256) else 0
             dg_part = torch.empty(chunks, B, U, H, dtype=torch.float32, device=device) if chunks else None
             d_g32 = torch.empty(B, U, H, dtype=torch.float32, device=device) if (want_g and not chunks) else None
             with torch.cuda.device(device):
