@@ -412,7 +412,7 @@ int mi_transducer_wait_lengths(const int64_t* words, void* stream);
 #define MI_PROFILE_DENOM 0   /* denom_rows_kernel / denom_block_kernel / denom_gather_kernel / joint_lse_kernel */
 #define MI_PROFILE_LATTICE 1 /* rnnt_lattice_kernel / tdt_lattice_pair_kernel / tdt_lattice_kernel */
 #define MI_PROFILE_CELL 2    /* rnnt_cell_kernel / tdt_cell_kernel */
-#define MI_PROFILE_GRAD 3    /* grad_rows_kernel / grad_block_kernel / grad_stream_kernel / joint_dhidden_kernel */
+#define MI_PROFILE_GRAD 3    /* grad_tile_kernel / grad_rows_kernel / grad_block_kernel / grad_stream_kernel / joint_dhidden_kernel */
 #define MI_PROFILE_ZERO 4    /* zero_padding_kernel */
 #define MI_PROFILE_DWEIGHT 5 /* joint_dweight_kernel */
 #define MI_PROFILE_KERNELS 6
@@ -425,7 +425,9 @@ int mi_transducer_profile_disable(void);
  * its coefficients itself).  D = 0 for RNNT; for TDT pass the largest duration; for the multi-blank
  * loss D = 0, num_big_blanks > 0 (V counting the big blanks) and max_duration the longest big blank.  Assumes a gradient
  * buffer at the 16-byte phase of the logits.  Launches nothing.  For benchmarks, profiles and tests
- * that want to name (or pin) the kernel family a shape maps to. */
+ * that want to name (or pin) the kernel family a shape maps to.  R=1 in a row kernel's name: rows of at most 64
+ * vectors, which denom_tile_kernel (RPW: the vectors a thread moves) and grad_tile_kernel (from 49 vectors on
+ * grad_rows_kernel) take. */
 int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D, int max_duration,
                                 int use_plain_rnnt, int num_big_blanks, char* out, size_t out_bytes);
 

@@ -280,6 +280,10 @@ inline RowTile row_tile(const PlanShape& s) {
 }
 inline int tile_chunks(const PlanShape& s, const RowTile& t) { return (s.U + t.rows() - 1) >> t.log_rows; }
 inline long long tile_blocks(const PlanShape& s, const RowTile& t) { return (long long)tile_chunks(s, t) * s.B * s.T; }
+// ... but for the gradient of rows that give nearly every lane of a wave its vector (grad_rows_kernel).
+inline bool grad_by_rows(const PlanShape& s) {
+  return MI_USE_ROWS && s.same_phase && s.whole_vectors() > 48 && s.whole_vectors() <= 64;
+}
 // Pass 1 over them: as many cells, but 16 (or a power of two that holds U) rows of each of several frames.
 constexpr int kTileMaxFrames = 16;
 struct DenomTile {

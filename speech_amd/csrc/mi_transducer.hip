@@ -13,7 +13,7 @@
 //   cells    tdt_cell_kernel | multiblank_cell_kernel | rnnt_cell_kernel (RNNT rows of more than 64 vectors: none, the gradient
 //            pass derives them itself)
 //            one thread per lattice cell: the few numbers a gradient row needs, grad_scale folded in.
-//   pass 2   grad_tile_kernel (mi_tile.inc) | grad_block_kernel | grad_stream_kernel   (mi_streaming.inc)
+//   pass 2   grad_tile_kernel (mi_tile.inc) | grad_rows_kernel | grad_block_kernel | grad_stream_kernel   (mi_streaming.inc)
 //            streams acts a second time and writes every gradient element once, zeros for padded cells included.
 // The compact log-prob op (mi_logprobs.inc) reuses pass 1 and pass 2; the fused joint + loss (mi_joint.inc) replaces
 // pass 1 and the producer of the logits by an MFMA kernel.  Host-side checks and launchers: mi_host.inc.
