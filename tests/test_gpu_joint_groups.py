@@ -1,11 +1,12 @@
 """The fused joint's forward kernel gives a wave 32 cells (few tiles) or 64 (many), and computes only the blocks of 64
-vocabulary rows that are in use: both splits against the loss on materialised logits, vocabularies around a block's edges."""
+vocabulary rows that are in use: both splits, for every loss and activation and with dropout, against the loss on
+materialised logits, vocabularies around a block's edges."""
 
 import pytest
 import torch
 
-from speech_amd import RNNTLossNumba
-from speech_amd.joint import joint_rnnt_loss
+from speech_amd import MultiblankRNNTLossNumba, RNNTLossNumba, TDTLossNumba
+from speech_amd.joint import joint_dropout_mask, joint_multiblank_loss, joint_rnnt_loss, joint_tdt_loss
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +49,50 @@ def test_both_splits(B, T, U, V, H):
     for name, got, ref in zip(("f", "g", "weight", "bias"), grads, want_grads):
         # gradient entries and d hidden are bf16 (2^-9 each, logits fp16): sums of them stay within 2^-6 of the largest
         assert (got - ref).abs().max() <= 2.0**-6 * ref.abs().max(), name
+
+
+# what one group and two groups of cells compile to for the other losses, activations and dropout; duration rows (from V on)
+# and big blanks (below the blank) on both sides of a block's edge
+@pytest.mark.parametrize("B,T,U", [(3, 21, 9), (9, 130, 57)])
+@pytest.mark.parametrize("loss,V,H", [("rnnt", 65, 640), ("tdt", 62, 640), ("tdt", 126, 512), ("tdt", 64, 320),
+                                      ("multiblank", 67, 640), ("multiblank", 131, 512), ("multiblank", 66, 256)])  # fmt: skip
+@pytest.mark.parametrize("activation,dropout", [("relu", 0.3), ("tanh", 0.0), ("sigmoid", 0.2)])
+def test_both_splits_of_every_loss_and_activation(B, T, U, loss, V, H, activation, dropout):
+    steps = {"rnnt": [], "tdt": [0, 1, 2, 3, 4], "multiblank": [2, 4, 8]}[loss]
+    rows = V + len(steps) if loss == "tdt" else V
+    leaves, rest = _inputs(B, T, U, rows, H, V + B + len(activation))
+    f, g, weight, bias = leaves
+    rest = (rest[0] % (V - 1 - len(steps)), *rest[1:])  # token ids only
+    options = dict(dropout=dropout, seed=99, activation=activation)
+    keep = joint_dropout_mask(B, T, U, H, dropout, 99, f.device) if dropout else None
+
+    def fused():
+        if loss == "tdt":
+            return joint_tdt_loss(f, g, weight, bias, *rest, V - 1, steps, sigma=0.05, **options)
+        if loss == "multiblank":
+            return joint_multiblank_loss(f, g, weight, bias, *rest, V - 1, steps, sigma=0.05, **options)
+        return joint_rnnt_loss(f, g, weight, bias, *rest, V - 1, **options)
+
+    module = {
+        "rnnt": lambda: RNNTLossNumba(blank=V - 1, reduction="none"),
+        "tdt": lambda: TDTLossNumba(blank=V - 1, durations=steps, reduction="none", sigma=0.05),
+        "multiblank": lambda: MultiblankRNNTLossNumba(blank=V - 1, big_blank_durations=steps, reduction="none", sigma=0.05),
+    }[loss]()
+
+    def rounded(x):  # to bf16 as the joint network's layers round under autocast; the gradient passes in float32
+        return x + (x.detach().to(torch.bfloat16).float() - x.detach())
+
+    def materialised():  # (a backward in bf16 would round at every layer: its error alone reaches the bound below)
+        hidden = rounded(getattr(torch, activation)(rounded(f.float().unsqueeze(2) + g.float().unsqueeze(1))))
+        if dropout:
+            hidden = rounded(hidden * keep / (1.0 - dropout))
+        return module(hidden @ rounded(weight).T + bias, *rest)
+
+    costs, grads = _grads(fused, leaves)
+    want, want_grads = _grads(materialised, leaves)
+    torch.testing.assert_close(costs, want, rtol=1e-5, atol=1e-3)
+    for name, got, ref in zip(("f", "g", "weight", "bias"), grads, want_grads):
+        # (the bound of the test above)
+        assert (got - ref).abs().max() <= 2.0**-6 * ref.abs().max(), name
+    if loss == "tdt":  # the duration rows on their own: small beside the token rows
+        assert (grads[2] - want_grads[2])[V:].abs().max() <= 2.0**-6 * want_grads[2][V:].abs().max()
