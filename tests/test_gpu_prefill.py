@@ -102,6 +102,25 @@ def test_riders_fill_padding_beside_a_long_lattice(kind):
     assert (~torch.isnan(after_forward)).any(), "the riders filled nothing beside a lattice of 340 anti-diagonals"
 
 
+# RNNT lattices of several waves: 8 and 16 a workgroup, riders of 512 and 1024 threads (U > 256, U > 512); up to U = 256
+# one wave beside riders and four without them
+@pytest.mark.parametrize("U,T,V", [(130, 250, 33), (200, 250, 70), (256, 90, 5), (257, 90, 29), (300, 250, 33), (512, 40, 9),
+                                   (513, 40, 9), (600, 150, 21), (1024, 60, 6)])  # fmt: skip
+def test_lattices_of_several_waves_beside_riders(U, T, V):
+    B = 5
+    acts, labels, al, ll = make(U, B, T, U, V, torch.float32)
+    al[:] = torch.tensor([T, 1, T // 3, 2 * T // 3, T // 2], device=DEV)
+    ll[:] = torch.tensor([63, U - 1, 0, min(127, U - 1), U // 2], device=DEV)  # labels that end at a wave's edge and beside it
+    c0, g0, _ = run("rnnt", acts, labels, al, ll, False)
+    ws = rnnt.new_workspace(acts)
+    c1, g1, after_forward = run("rnnt", acts, labels, al, ll, True, ws=ws)
+    assert torch.isfinite(c0).all() and torch.isfinite(g0).all()
+    assert torch.equal(c0, c1) and torch.equal(g0, g1)
+    check_forward_touched_padding_only(after_forward, al, ll, ws)
+    if T + U > 400:
+        assert (~torch.isnan(after_forward)).any(), "the riders filled nothing beside a lattice of several hundred diagonals"
+
+
 @pytest.mark.parametrize("kind", ["rnnt", "tdt", "multiblank"])
 @pytest.mark.parametrize("junk", ["nan", "ff", "zero"])
 def test_junk_in_the_workspace_does_not_reach_the_result(kind, junk):
