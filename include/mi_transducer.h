@@ -425,9 +425,7 @@ int mi_transducer_profile_disable(void);
  * its coefficients itself).  D = 0 for RNNT; for TDT pass the largest duration; for the multi-blank
  * loss D = 0, num_big_blanks > 0 (V counting the big blanks) and max_duration the longest big blank.  Assumes a gradient
  * buffer at the 16-byte phase of the logits.  Launches nothing.  For benchmarks, profiles and tests
- * that want to name (or pin) the kernel family a shape maps to.  R=1 in a row kernel's name: rows of at most 64
- * vectors, which denom_tile_kernel (RPW: the vectors a thread moves) and grad_tile_kernel (from 49 vectors on
- * grad_rows_kernel) take. */
+ * that want to name (or pin) the kernel family a shape maps to. */
 int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D, int max_duration,
                                 int use_plain_rnnt, int num_big_blanks, char* out, size_t out_bytes);
 

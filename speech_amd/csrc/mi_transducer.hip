@@ -553,8 +553,10 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   char denom[96], lattice[96], cells[48], grad[112];
   const BlockPlan dp = denom_block_plan(c);
   if (dp.RT) snprintf(denom, sizeof denom, "denom_block_kernel<%s, RT=%d, NVT=%d>", dt, dp.RT, dp.NVT);
-  // R=1: short rows, the tile kernels of mi_tile.inc (RPW: the vectors of a tile a thread moves)
-  else if (row_tile(c).log_rows) snprintf(denom, sizeof denom, "denom_rows_kernel<%s, R=1, RPW=%d>", dt, kTileRounds);
+  else if (row_tile(c).log_rows) {
+    const DenomTile tile = denom_tile(shape_of(c));
+    snprintf(denom, sizeof denom, "denom_tile_kernel<%s, rows=%d, frames=%d>", dt, 1 << tile.log_rows, 1 << tile.log_frames);
+  }
   else if (denom_rows_R(c)) snprintf(denom, sizeof denom, "denom_rows_kernel<%s, R=%d, RPW=%d>", dt, denom_rows_R(c), denom_rows_per_wave(denom_rows_R(c)));
   else snprintf(denom, sizeof denom, "denom_gather_kernel<%s>", dt);
   const bool tdt = D > 0 && !use_plain_rnnt;
@@ -577,7 +579,8 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   const bool fused = !tdt && !mb && rnnt_rows_fused(c, nullptr);
   snprintf(cells, sizeof cells, "%s", fused ? "-" : (mb ? "multiblank_cell_kernel" : (tdt ? "tdt_cell_kernel" : "rnnt_cell_kernel")));
   if (gp.RT) snprintf(grad, sizeof grad, "grad_block_kernel<%s, RT=%d, NVT=%d, %s>", dt, gp.RT, gp.NVT, fused ? "fused" : "coef");
-  else if (row_tile(c).log_rows) snprintf(grad, sizeof grad, "grad_rows_kernel<%s, R=1, coef>", dt);
+  else if (grad_by_rows(shape_of(c))) snprintf(grad, sizeof grad, "grad_rows_kernel<%s>", dt);
+  else if (row_tile(c).log_rows) snprintf(grad, sizeof grad, "grad_tile_kernel<%s, rows=%d>", dt, row_tile(c).rows());
   else snprintf(grad, sizeof grad, "grad_stream_kernel<%s>", dt);
   const int n = snprintf(out, out_bytes, "denominators=%s; lattice=%s; cells=%s; gradient=%s%s", denom, lattice, cells,
                          grad, (mb && !gp.RT) ? " + multiblank_fixup_kernel" : "");

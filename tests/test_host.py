@@ -67,7 +67,7 @@ def test_kernel_plan_of_the_documented_shapes(built_lib):
     assert p["denominators"] == "denom_block_kernel<f32, RT=1024, NVT=4>"
     assert p["gradient"] == "grad_block_kernel<f32, RT=1024, NVT=4, fused>"
     p = plan(F32, 4, 50, 21, 29)  # character vocabulary: short rows, coefficients from the cell kernel
-    assert p["denominators"] == "denom_rows_kernel<f32, R=1, RPW=4>" and p["gradient"] == "grad_rows_kernel<f32, R=1, coef>"
+    assert p["denominators"] == "denom_tile_kernel<f32, rows=16, frames=8>" and p["gradient"] == "grad_tile_kernel<f32, rows=32>"
     assert p["cells"] == "rnnt_cell_kernel"
     p = plan(F32, 2, 10, 5, 40001)  # beyond 8 vectors per thread: the streaming kernels with a running max
     assert p["denominators"] == "denom_gather_kernel<f32>" and p["gradient"] == "grad_stream_kernel<f32>"
@@ -84,8 +84,8 @@ def test_kernel_plan_of_the_documented_shapes(built_lib):
     assert p["denominators"] == "denom_rows_kernel<f32, R=5, RPW=1>"
     # (that kernel writes the big blanks' entries itself; only the other gradient kernels are followed by a fix-up)
     assert p["gradient"] == "grad_block_kernel<f32, RT=128, NVT=3, coef>"
-    p = plan(F32, 4, 50, 21, 32, num_big_blanks=3)  # short rows: the wave-per-row kernel, then the fix-up kernel
-    assert p["gradient"] == "grad_rows_kernel<f32, R=1, coef> + multiblank_fixup_kernel"
+    p = plan(F32, 4, 50, 21, 32, num_big_blanks=3)  # short rows: the tile kernel, then the fix-up kernel
+    assert p["gradient"] == "grad_tile_kernel<f32, rows=32> + multiblank_fixup_kernel"
     p = plan(F32, 2, 50, 1024, 1028, max_duration=8, num_big_blanks=3)  # ring of 9 x 6 x 1024 doubles > 160 KB of LDS
     assert p["lattice"] == "multiblank_lattice_pull_kernel"
     p = plan(F32, 2, 50, 513, 1025, D=9, max_duration=8)  # beyond 256 label columns: a wave per direction
@@ -94,6 +94,20 @@ def test_kernel_plan_of_the_documented_shapes(built_lib):
         plan(7, 1, 1, 1, 5)
     with pytest.raises(RuntimeError):
         plan(F32, 1, 4, 2, 9, D=2, max_duration=1, num_big_blanks=2)  # TDT and multi-blank exclude each other
+
+
+def test_kernel_plan_of_rows_about_64_vectors(built_lib):
+    """Tiles up to 64 whole vectors, whole waves a row from 65 on; the gradient of 49 to 64 vectors takes a wave a row."""
+    for dtype, name, vec in [(0, "f32", 4), (1, "bf16", 8), (2, "f16", 8)]:
+        for vectors in (1, 16, 48, 49, 64, 65):
+            for V in (vectors * vec, vectors * vec + vec - 1):
+                p = _native.describe_plan(dtype, 16, 375, 121, V)
+                denominators, gradient = p["denominators"].split("<")[0], p["gradient"].split("<")[0]
+                assert f"<{name}" in p["denominators"] and f"<{name}" in p["gradient"]
+                assert denominators == ("denom_tile_kernel" if vectors <= 64 else "denom_rows_kernel"), V
+                by_rows = 48 < vectors <= 64
+                assert gradient == ("grad_block_kernel" if vectors > 64 else "grad_rows_kernel" if by_rows else "grad_tile_kernel"), V
+                assert p["cells"] == ("rnnt_cell_kernel" if vectors <= 64 else "-")
 
 
 def test_constructor_attributes_match_the_reference_conventions():
