@@ -280,9 +280,17 @@ inline RowTile row_tile(const PlanShape& s) {
 }
 inline int tile_chunks(const PlanShape& s, const RowTile& t) { return (s.U + t.rows() - 1) >> t.log_rows; }
 inline long long tile_blocks(const PlanShape& s, const RowTile& t) { return (long long)tile_chunks(s, t) * s.B * s.T; }
-// ... but for the gradient of rows that give nearly every lane of a wave its vector (grad_rows_kernel).
+// ... but for the gradient of 16-bit rows that give nearly every lane of a wave its vector (grad_rows_kernel): eight elements
+// a vector, and a tile selects each element's coefficients (and looks for duration entries among them), which are
+// wave-uniform there.  A float32 vector has half the selects for the same bytes, and tiles win.  Measured, step at B=16,
+// T=375, U=121 (us, tiles / a wave a row), by whole vectors:
+//   RNNT float32 49 279 / 309, 56 295 / 326, 64 322 / 353; bfloat16 36 276 / 310, 49 324 / 330, 56 345 / 345, 60 357 / 352,
+//   64 373 / 370; multi-blank bfloat16 49 479 / 489, 56 500 / 506
+//   TDT  float32 49 490 / 515, 64 535 / 564; 16 bits, five durations 34 511 / 519, 40 540 / 530, 48 571 / 543, 56 606 / 561,
+//   two durations 34 425 / 444, 40 451 / 457, 44 463 / 462, 48 483 / 473
 inline bool grad_by_rows(const PlanShape& s) {
-  return MI_USE_ROWS && s.same_phase && s.whole_vectors() > 48 && s.whole_vectors() <= 64;
+  const int nb = s.whole_vectors();
+  return MI_USE_ROWS && s.same_phase && s.vec() == 8 && nb > (s.D ? 40 : 56) && nb <= 64;
 }
 // Pass 1 over them: as many cells, but 16 (or a power of two that holds U) rows of each of several frames.
 constexpr int kTileMaxFrames = 16;

@@ -49,6 +49,26 @@ def test_rnnt(U, V, dtype):
     _check(_run(loss, x, *rest), want, dtype)
 
 
+# 16-bit rows of 57 to 64 vectors, with durations 41 to 64, give their gradient a wave each: the last rows of the tiles and
+# the first of the waves, the same rows in float32
+@pytest.mark.parametrize("V", [455, 456, 512])
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+def test_rnnt_rows_about_the_line(V, dtype):
+    x, *rest = _case(11, V, dtype)
+    loss = RNNTLossNumba(blank=V - 1, reduction="none", fastemit_lambda=0.01, clamp=0.4)
+    want = oracle.rnnt_loss(x.double().numpy(), *rest, V - 1, 0.01, 0.4)
+    _check(_run(loss, x, *rest), want, dtype)
+
+
+@pytest.mark.parametrize("V,dtype", [(327, BF16), (328, BF16), (335, torch.float16), (515, BF16), (197, F32), (255, F32)])
+def test_tdt_rows_about_the_line(V, dtype):
+    durations = [0, 1, 2, 3, 4]
+    x, *rest = _case(11, V, dtype, extra=len(durations))
+    loss = TDTLossNumba(blank=V - 1, durations=durations, reduction="none", sigma=0.05)
+    want = oracle.tdt_loss(x.double().numpy(), *rest, V - 1, durations, 0.05)
+    _check(_run(loss, x, *rest), (want[0], want[1]), dtype)
+
+
 @pytest.mark.parametrize("U,V", [(9, 3), (65, 29), (16, 129), (8, 257)])
 @pytest.mark.parametrize("dtype", [F32, BF16])
 def test_tdt(U, V, dtype):

@@ -97,17 +97,18 @@ def test_kernel_plan_of_the_documented_shapes(built_lib):
 
 
 def test_kernel_plan_of_rows_about_64_vectors(built_lib):
-    """Tiles up to 64 whole vectors, whole waves a row from 65 on; the gradient of 49 to 64 vectors takes a wave a row."""
+    """Tiles up to 64 whole vectors, whole waves a row from 65 on; the gradient of 57 (with durations 41) to 64 vectors in
+    16 bits takes a wave a row."""
     for dtype, name, vec in [(0, "f32", 4), (1, "bf16", 8), (2, "f16", 8)]:
-        for vectors in (1, 16, 48, 49, 64, 65):
-            for V in (vectors * vec, vectors * vec + vec - 1):
-                p = _native.describe_plan(dtype, 16, 375, 121, V)
+        for vectors in (1, 16, 40, 41, 56, 57, 64, 65):
+            for V, D in [(vectors * vec, 0), (vectors * vec + vec - 1, 0), (vectors * vec + vec - 1, 5)]:
+                p = _native.describe_plan(dtype, 16, 375, 121, V, D=D, max_duration=4 if D else 0)
                 denominators, gradient = p["denominators"].split("<")[0], p["gradient"].split("<")[0]
                 assert f"<{name}" in p["denominators"] and f"<{name}" in p["gradient"]
                 assert denominators == ("denom_tile_kernel" if vectors <= 64 else "denom_rows_kernel"), V
-                by_rows = 48 < vectors <= 64
+                by_rows = vec == 8 and (40 if D else 56) < vectors <= 64
                 assert gradient == ("grad_block_kernel" if vectors > 64 else "grad_rows_kernel" if by_rows else "grad_tile_kernel"), V
-                assert p["cells"] == ("rnnt_cell_kernel" if vectors <= 64 else "-")
+                assert p["cells"] == ("tdt_cell_kernel" if D else "rnnt_cell_kernel" if vectors <= 64 else "-")
 
 
 def test_constructor_attributes_match_the_reference_conventions():
