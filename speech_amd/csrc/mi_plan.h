@@ -27,8 +27,9 @@ constexpr int kFillMaxRiders = 4096;
 constexpr int kFillProgress = 2 * kFillMaxLattice;
 constexpr int kFillInts = kFillProgress + kFillMaxRiders;
 constexpr int kFillLogRowsShift = 8;  // the gradient kernels find log2(rows per item) in these bits of `flags`
-// Rows per item: eight (no workgroup of the gradient pass spans more rows, and none straddles a multiple of eight),
-// fewer for long rows, so that a rider looks at the lattice's state every 64 KB or so
+// Rows per item: eight (the gradient kernels that look at one item span no more rows and straddle no multiple of eight; a
+// tile of short rows looks at up to 16 items), fewer for long rows, so that a rider looks at the lattice's state every 64
+// KB or so
 inline int prefill_log_rows(size_t row_bytes) {
   int log_rows = 3;
   while (log_rows > 0 && (row_bytes << log_rows) > 64 * 1024) --log_rows;
@@ -196,17 +197,10 @@ struct PlanShape {
 #endif
 constexpr int kRowWaves = MI_ROW_WAVES;  // waves (= rows in flight) per workgroup of the row kernels
 
-// smallest R in {1,2,4,8} with floor(V / VEC) <= 64*R, or 0 if the rows are too long for the
-// register-resident kernels
-inline int rows_R(const PlanShape& s) {
-  if (!MI_USE_ROWS) return 0;
-  const int nb = s.whole_vectors();
-  for (int r = 1; r <= 8; r *= 2)
-    if (nb <= 64 * r) return r;
-  return 0;
-}
-// The denominator pass may take R = 3, 5, 6 as well: a vocabulary just past a power of two -- 1024 tokens, the
-// blank and three big blanks are 257 vectors -- then costs 5 vector loads per lane, not 8.
+// Pass 1 of rows beyond 64 vectors, a wave per row: the smallest R of these with floor(V / VEC) <= 64*R, or 0 if the rows are
+// too long for the register-resident kernels.
+// (3, 5 and 6 as well: a vocabulary just past a power of two -- 1024 tokens, the blank and three big blanks are 257 vectors
+// -- then costs 5 vector loads per lane, not 8)
 inline int denom_rows_R(const PlanShape& s) {
   if (!MI_USE_ROWS) return 0;
   const int nb = s.whole_vectors();
@@ -214,8 +208,6 @@ inline int denom_rows_R(const PlanShape& s) {
     if (r != 7 && nb <= 64 * r) return r;
   return 0;
 }
-// the row kernels store gradient vectors at the 16-byte phase of the logits row
-inline int grad_rows_R(const PlanShape& s) { return s.same_phase ? rows_R(s) : 0; }
 
 // Workgroup-per-row kernels: RT threads per row, NVT vectors per thread.  RT == 0: not applicable.
 // The denominator pass uses them for rows too long for the register-resident wave-per-row
@@ -267,6 +259,9 @@ inline long long row_blocks(const PlanShape& s, int rpw) { return (long long)row
 // on every lane has work there (measured figures: mi_tile.inc).
 constexpr int kTileBytes = 17 * 1024 - 16;
 constexpr int kTileMaxRows = 128;
+constexpr int kTileThreads = 256;
+constexpr int kTileRounds = (kTileBytes + 16) / 16 / kTileThreads;  // aligned vectors a thread moves; a few move one more
+static_assert(kTileRounds == 4, "a tile is four vectors a thread, and some");
 struct RowTile {
   int log_rows;  // 0: not a short row
   int rows() const { return 1 << log_rows; }
@@ -294,6 +289,10 @@ inline bool grad_by_rows(const PlanShape& s) {
 }
 // Pass 1 over them: as many cells, but 16 (or a power of two that holds U) rows of each of several frames.
 constexpr int kTileMaxFrames = 16;
+// the pieces of a tile's frames each start and end inside a vector
+constexpr int kTileVectors = kTileBytes / 16 + 2 * kTileMaxFrames;
+// elements of a row a lane reduces (rows * V elements over the workgroup's threads, four at a time)
+constexpr int tile_share(int element_bytes) { return (kTileBytes / element_bytes / kTileThreads + 4) / 4 * 4; }
 struct DenomTile {
   int log_rows, log_frames;  // log_rows + log_frames: 3 ... 7
   int frame_groups;          // groups of frames per utterance
@@ -309,7 +308,6 @@ inline DenomTile denom_tile(const PlanShape& s) {
   while (d.log_rows < 4 && d.log_rows < log_cells && (1 << d.log_rows) < s.U) ++d.log_rows;
   d.log_frames = log_cells - d.log_rows;
   if ((1 << d.log_frames) > kTileMaxFrames) d.log_frames = 4;
-  if (d.log_rows + d.log_frames < 3) d.log_frames = 3 - d.log_rows;
   d.frame_groups = (s.T + (1 << d.log_frames) - 1) >> d.log_frames;
   d.pitch = (int)(((row_bytes << d.log_rows) + 15) / 16) + 1;
   d.div_pitch = make_fastdiv((unsigned)d.pitch);

@@ -43,6 +43,37 @@ static int failures = 0;
     }                                                      \
   } while (0)
 
+// Tiles of short rows: what the kernels of mi_tile.inc rely on to stay inside their LDS, registers and grid.
+static void fuzz_tiles(const PlanShape& s) {
+  const RowTile t = row_tile(s);
+  EXPECT((t.log_rows != 0) == (s.whole_vectors() <= 64), "short row V %d", s.V);
+  if (grad_by_rows(s)) EXPECT(t.log_rows && s.same_phase && s.vec() == 8, "a wave per row V %d", s.V);
+  if (!t.log_rows) return;
+  const long long element = 16 / s.vec(), row_bytes = (s.V + s.D) * element;
+  const long long moved = kTileThreads * (kTileRounds + 1);  // vectors a workgroup can move
+  EXPECT(t.rows() >= 8 && t.rows() <= kTileMaxRows && t.rows() <= kTileThreads, "rows %d", t.rows());
+  EXPECT(row_bytes * t.rows() / 16 + 1 <= moved, "gradient tile rows %d V %d D %d", t.rows(), s.V, s.D);
+  EXPECT(t.rows() >> prefill_log_rows((size_t)row_bytes) <= 16, "prefill items of a tile, rows %d V %d", t.rows(), s.V);
+  EXPECT((long long)tile_chunks(s, t) * t.rows() >= s.U && (long long)(tile_chunks(s, t) - 1) * t.rows() < s.U, "chunks cover U");
+  const DenomTile d = denom_tile(s);
+  const int log_cells = d.log_rows + d.log_frames, lanes = kTileThreads >> log_cells, slots = d.pitch << d.log_frames;
+  EXPECT(log_cells >= 3 && (1 << log_cells) <= kTileMaxRows && lanes >= 2 && lanes <= 64 && (1 << d.log_frames) <= kTileMaxFrames,
+         "denominator tile rows %d frames %d", 1 << d.log_rows, 1 << d.log_frames);
+  EXPECT(slots <= kTileVectors && slots <= moved, "slots %d V %d D %d U %d", slots, s.V, s.D, s.U);
+  EXPECT((long long)d.pitch * 16 >= (row_bytes << d.log_rows) + 16 - element, "pitch %d", d.pitch);
+  EXPECT(lanes * tile_share((int)element) >= s.V, "share of a lane, V %d lanes %d", s.V, lanes);
+  for (int i = 0; i < slots; ++i) {
+    const unsigned q = (unsigned)(((((unsigned long long)i * d.div_pitch.mul) >> 32) + i) >> d.div_pitch.shift);
+    EXPECT(q == (unsigned)i / (unsigned)d.pitch, "slot %d of pitch %d", i, d.pitch);
+  }
+  EXPECT((long long)d.frame_groups << d.log_frames >= s.T && (long long)(d.frame_groups - 1) << d.log_frames < s.T, "frames");
+  EXPECT((long long)denom_tile_chunks(s, d) << d.log_rows >= s.U, "rows");
+  for (const long long blocks : {tile_blocks(s, t), denom_tile_blocks(s, d)}) {
+    const unsigned turn = 8u << tile_log_span(blocks);
+    EXPECT(tile_grid(blocks) >= blocks && tile_grid(blocks) < blocks + turn && tile_grid(blocks) % turn == 0, "grid");
+  }
+}
+
 static void fuzz_plan(std::mt19937& rng, int iterations) {
   auto uni = [&](int lo, int hi) { return std::uniform_int_distribution<int>(lo, hi)(rng); };
   for (int it = 0; it < iterations; ++it) {
@@ -106,12 +137,13 @@ static void fuzz_plan(std::mt19937& rng, int iterations) {
     if (ms == MI_TRANSDUCER_SUCCESS) EXPECT(mp.R == longest + 1, "ring depth");
     // kernel shapes: whatever is chosen must cover the row and fit a workgroup
     PlanShape s;
-    s.dt = uni(0, 2); s.B = uni(1, 64); s.T = uni(1, 800); s.U = uni(1, 1024); s.V = uni(1, 70000); s.D = uni(0, 16);
+    s.dt = uni(0, 2); s.B = uni(1, 64); s.T = uni(1, 800); s.U = uni(1, uni(0, 1) ? 1024 : 40);
+    s.V = uni(1, uni(0, 1) ? 70000 : 530); s.D = uni(0, 16);
     s.same_phase = uni(0, 3) != 0;
     const int nb = s.whole_vectors();
-    const int r1 = denom_rows_R(s), r4 = grad_rows_R(s);
+    const int r1 = denom_rows_R(s);
     if (r1) EXPECT(nb <= 64 * r1 && r1 <= 8 && r1 != 7, "denominator rows R %d nb %d", r1, nb);
-    if (r4) EXPECT(nb <= 64 * r4 && s.same_phase, "gradient rows R %d nb %d", r4, nb);
+    fuzz_tiles(s);
     const BlockPlan dp = denom_block_plan(s), gp = grad_block_plan(s);
     if (dp.RT) EXPECT(dp.RT == 1024 && nb > 512 && nb <= dp.RT * dp.NVT && dp.NVT <= 8, "denominator block plan");
     if (gp.RT) {
