@@ -433,7 +433,7 @@ def run_joint(args, torch, dev, cfg, labels, act_lens, label_lens):
         "config": {"workload": cfg.name.replace("_f32", "") + "_joint_H%d_bf16" % H, "B": B, "T": T, "U": U, "V": V, "H": H,
                    "valid_cells": valid, "cells": B * T * U},
         "roofline": {
-            "kernel": "joint_lse_kernel<H=%d> (the longest of the three product kernels)" % H, "bound": "mfma",
+            "kernel": "joint_lse_kernel<H=%d> (the forward product)" % H, "bound": "mfma",
             "achieved": achieved, "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / MFMA_BF16_PEAK_TFLOPS,
             "traffic": None, "algorithmic_flops_per_launch": flops, "avg_launch_ms": fwd_s * 1e3,
             "launches": kernels["denominator_pass"][1],

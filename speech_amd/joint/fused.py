@@ -293,9 +293,11 @@ class JointRNNTLoss(torch.autograd.Function):
             d_f32 = torch.empty(B, T, H, dtype=torch.float32, device=device) if want_f else None
             # both wanted (the usual case): one pass over d_hidden forms d f and, per run of frames, a share of d g (runs
             # of a length that U alone decides: the sums then do not depend on how a batch is split into sub-batches).
-            # A workgroup walks its run frame by frame, a barrier each; where a frame is short (U <= 64) its latency is
-            # the bound and runs of 16 frames are faster than runs of 32: B=4, T=190, U=49 48 -> 27 us, B=8, T=250, U=60
-            # 52 -> 49 us.  Longer frames keep 32, and half the partial sums.
+            # A workgroup walks its run frame by frame, a barrier each: shorter runs give more workgroups, longer ones
+            # fewer partial sums to add.  Runs of 16 frames against 32, us: the reduction at B=4, T=190, U=49, H=640
+            # 27 / 48; a step at B=16, T=375, H=640, V=257: U=33 472 / 469, U=64 710 / 703, U=121 1139 / 1138.  Few
+            # utterances gain from 16 at larger U too (B=8, T=250, H=256: U=96 270 / 289, U=121 306 / 331), but their
+            # number must not decide.
             run = 16 if U <= 64 else 32
             chunks = (T + run - 1) // run if (want_f and want_g and U <= 256) else 0
             dg_part = torch.empty(chunks, B, U, H, dtype=torch.float32, device=device) if chunks else None
