@@ -176,6 +176,51 @@ inline int make_mb_params(int NB, const int32_t* durations, float sigma, MbParam
 
 
 // ----------------------------------------------------------------------------------------
+// Lattices on probabilities (mi_scaled.inc)
+// ----------------------------------------------------------------------------------------
+constexpr int kScaledMaxGroups = 4;  // 256 columns
+// doubles per cell that a helper leaves in LDS: TDT the two tokens and durations 0 .. maxd, multi-blank the label and the
+// blanks of duration 1 .. maxd; in whole pairs, the last of them free
+constexpr int scaled_factors(bool tdt, int maxd) { return ((tdt ? 3 + maxd : 1 + maxd) + 1) / 2 * 2; }
+constexpr size_t scaled_group_bytes(int factors, int steps) { return (size_t)steps * (1024 * (factors + 1) + 176); }
+struct ScaledPlan {
+  int longest;  // the longest duration the instantiation holds: 4 or 8; 0: the recursions on logarithms
+  int steps;    // anti-diagonals a batch
+  int helpers;  // helper waves per group of 64 columns
+  int threads;
+  size_t lds;
+};
+// Batches of 8 diagonals and four helpers a group, as far as LDS holds them and for one or two groups; beyond, batches of 4,
+// and two helpers: four groups then have the twelve waves that a compute unit gives enough registers.
+// longest == 0: longer durations, more than 256 columns (192 with a longest duration above 4), more LDS than there is.
+inline ScaledPlan scaled_plan(bool tdt, int longest, int U) {
+  const int groups = (U + 63) / 64, maxd = longest <= 4 ? 4 : 8, factors = scaled_factors(tdt, maxd);
+  ScaledPlan p{0, 0, 0, 0, 0};
+  if (longest > 8 || groups > kScaledMaxGroups) return p;
+  for (int steps = 8; steps >= 4; steps -= 4) {
+    const size_t lds = groups * scaled_group_bytes(factors, steps) + 16;
+    if (lds > 160 * 1024 || (steps == 8 && groups > 2)) continue;
+    const int helpers = groups > 2 ? 2 : 4;
+    return ScaledPlan{maxd, steps, helpers, 64 * groups * (1 + helpers), lds};
+  }
+  return p;
+}
+// offsets into an utterance's records are 32-bit (and run up to 256 diagonals past its end)
+inline bool scaled_offsets_fit(const Layout& L) { return (L.ND + 256LL) * L.Us * L.A * 4 < (1LL << 31); }
+inline ScaledPlan scaled_plan(const Layout& L, const TdtParams& p, int U) {
+  return scaled_offsets_fit(L) ? scaled_plan(true, p.dur[p.D - 1], U) : ScaledPlan{0, 0, 0, 0, 0};
+}
+// (a blank arc has a factor of its own per duration: the big blanks' durations must differ, also from the standard blank's)
+inline ScaledPlan scaled_plan(const Layout& L, const MbParams& p, int U) {
+  bool distinct = p.NB > 0 && scaled_offsets_fit(L);
+  for (int i = 0; i < p.NB; ++i) {
+    distinct = distinct && p.dur[i] >= 2;
+    for (int j = 0; j < i; ++j) distinct = distinct && p.dur[j] != p.dur[i];
+  }
+  return distinct ? scaled_plan(false, p.R - 1, U) : ScaledPlan{0, 0, 0, 0, 0};
+}
+
+// ----------------------------------------------------------------------------------------
 // Kernel shape per problem shape.  The shape of a call as far as these choices go: logit dtype, tokens per row,
 // extra row entries (TDT durations), lattice dimensions, and whether logits and gradients share their 16-byte phase.
 // ----------------------------------------------------------------------------------------

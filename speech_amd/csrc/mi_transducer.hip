@@ -6,8 +6,9 @@
 //            cell the denominator and, as one record of consecutive floats, the blank / label (/ duration /
 //            big-blank) log-probabilities, the records in a SKEWED layout [b][t+u][u][record], so that an
 //            anti-diagonal of the lattice is contiguous and a cell's record leaves in one store.
-//   lattice  rnnt_lattice_kernel | tdt_lattice_pair_kernel | tdt_lattice_kernel  (mi_lattice.inc)
-//            | multiblank_lattice_kernel | multiblank_lattice_pull_kernel        (mi_multiblank.inc)
+//   lattice  rnnt_lattice_kernel | tdt_lattice_ring_kernel | tdt_lattice_kernel  (mi_lattice.inc)
+//            | multiblank_lattice_ring_kernel | multiblank_lattice_pull_kernel   (mi_multiblank.inc)
+//            | tdt_lattice_pair_kernel | multiblank_lattice_kernel               (mi_scaled.inc)
 //            alpha and beta over the anti-diagonals, accumulated in fp64 (only the log1p(exp(.)) term in fp32);
 //            the alpha side writes costs.
 //   cells    tdt_cell_kernel | multiblank_cell_kernel | rnnt_cell_kernel (RNNT rows of more than 64 vectors: none, the gradient
@@ -55,6 +56,7 @@ namespace {
 #include "mi_lattice.inc"
 #include "mi_logprobs.inc"
 #include "mi_multiblank.inc"
+#include "mi_scaled.inc"
 #include "mi_streaming.inc"
 #include "mi_tile.inc"
 #include "mi_host.inc"
@@ -564,14 +566,16 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   if (mb) {
     const int nbc = num_big_blanks <= 1 ? 1 : (num_big_blanks <= 2 ? 2 : (num_big_blanks <= 4 ? 4 : 8));
     const size_t lds = (size_t)(max_duration + 1) * (2 + nbc) * c.L.Us * sizeof(double);
-    if (lds > 160 * 1024) snprintf(lattice, sizeof lattice, "multiblank_lattice_pull_kernel");
-    else snprintf(lattice, sizeof lattice, "multiblank_lattice_kernel<NBC=%d>", nbc);
+    if (scaled_plan(false, max_duration, U).longest) snprintf(lattice, sizeof lattice, "multiblank_lattice_kernel<NBC=%d>", nbc);
+    else if (lds > 160 * 1024) snprintf(lattice, sizeof lattice, "multiblank_lattice_pull_kernel");
+    else snprintf(lattice, sizeof lattice, "multiblank_lattice_ring_kernel<NBC=%d>", nbc);
   } else if (D == 0 || use_plain_rnnt) {
     snprintf(lattice, sizeof lattice, "rnnt_lattice_kernel<K=%d>", c.L.K);
   } else {
     const int R = max_duration + 2;
     const size_t lds_block = (size_t)R * 2 * D * c.L.Us * sizeof(double);
-    if (D <= 8 && c.L.Us <= 256 && lds_block <= 160 * 1024) snprintf(lattice, sizeof lattice, "tdt_lattice_pair_kernel<D=%d>", D);
+    if (scaled_plan(true, max_duration, U).longest) snprintf(lattice, sizeof lattice, "tdt_lattice_pair_kernel<D=%d>", D);
+    else if (D <= 8 && c.L.Us <= 256 && lds_block <= 160 * 1024) snprintf(lattice, sizeof lattice, "tdt_lattice_ring_kernel<D=%d>", D);
     else snprintf(lattice, sizeof lattice, "tdt_lattice_kernel<K=%d>", c.L.K);
   }
   // a gradient buffer at the 16-byte phase of the logits is assumed (what every allocator returns)
