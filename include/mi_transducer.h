@@ -366,6 +366,18 @@ int mi_joint_reduce_hidden(const void* d_hidden, const void* f, const void* g, c
                            float dropout_p, unsigned long long dropout_seed, int activation, int B, int T, int U, int H,
                            int V, int D, int num_big_blanks, void* workspace, size_t workspace_bytes, void* stream);
 
+/* Backward of the fused joint, the same last step together with the sums over the partial sums, every gradient in the dtype
+ * its caller wants (MI_DTYPE_*, entries rounded once from float32): with d_hidden != NULL the one pass over it (d_f [B,T,H]
+ * and dg_part as above, all of d_f, dg_part and d_g set) and d_g [B,U,H] = the sum of dg_part; d_weight [V+D,H] (or NULL) =
+ * the sum of dw_part over its `slices`, d_bias [V+D] (or NULL) the sum of db_part, both as the backward call left them.
+ * Every pointer is 16-byte aligned. */
+int mi_joint_gradient_sums(const void* d_hidden, const void* f, const void* g, const int64_t* act_lens,
+                           const int64_t* label_lens, void* d_f, int d_f_dtype, float* dg_part, int chunks, void* d_g,
+                           int d_g_dtype, const float* dw_part, const float* db_part, int slices, void* d_weight,
+                           int d_weight_dtype, void* d_bias, int d_bias_dtype, int tiles, float dropout_p,
+                           unsigned long long dropout_seed, int activation, int B, int T, int U, int H, int V, int D,
+                           int num_big_blanks, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Where the forward call left the packed weights inside its workspace: *rows x *pitch bf16, row n = weight[n, :]
  * followed by the bias columns (rows beyond V + D are zero in the first H columns), so that the d_hidden product
  * can read them in place. */

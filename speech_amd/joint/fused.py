@@ -33,7 +33,7 @@ import random
 import torch
 
 from speech_amd import _native
-from speech_amd.rnnt_loss.rnnt import _durations_array, _labels_ptr, _ptr, _require_gpu, _stream
+from speech_amd.rnnt_loss.rnnt import _DTYPE_CODE, _durations_array, _labels_ptr, _ptr, _require_gpu, _stream
 
 __all__ = ["joint_rnnt_forward", "joint_rnnt_loss", "joint_tdt_forward", "joint_tdt_loss", "joint_multiblank_forward",
            "joint_multiblank_loss", "joint_dropout_mask", "JointRNNTLoss"]  # fmt: skip
@@ -82,6 +82,11 @@ def _activation_code(activation):
     except KeyError:
         # the reference's message (modules/rnnt.py:1763)
         raise ValueError("Unsupported activation for joint step - please pass one of [relu, sigmoid, tanh]") from None
+
+
+def _sum_dtype(dtype):
+    """The dtype the kernels leave a gradient in: its own, or float32 for one they do not write."""
+    return dtype if dtype in _DTYPE_CODE else torch.float32
 
 
 def _draw_seed(dropout, seed):
@@ -283,37 +288,51 @@ class JointRNNTLoss(torch.autograd.Function):
                         _stream(device),
                     )  # fmt: skip
             _native.check_status(status, "fused joint backward")
-        if want_w:
+        want_f, want_g = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+        # Both of d f and d g wanted (the usual case): one pass over d_hidden forms d f and, per run of frames, a share of d g
+        # (runs of a length that U alone decides: the sums then do not depend on how a batch is split into sub-batches).
+        # A workgroup walks its run frame by frame, a barrier each: shorter runs give more workgroups, longer ones
+        # fewer partial sums to add.  Runs of 16 frames against 32, us: the reduction at B=4, T=190, U=49, H=640
+        # 27 / 48; a step at B=16, T=375, H=640, V=257: U=33 472 / 469, U=64 710 / 703, U=121 1139 / 1138.  Few
+        # utterances gain from 16 at larger U too (B=8, T=250, H=256: U=96 270 / 289, U=121 306 / 331), but their
+        # number must not decide.
+        run = 16 if U <= 64 else 32
+        one_pass = want_f and want_g and U <= 256
+        chunks = (T + run - 1) // run if one_pass else 0
+        if one_pass or want_w:
+            f_dtype, g_dtype = (_sum_dtype(t) for t in ctx.in_dtypes)
+            if one_pass:
+                d_f = torch.empty(B, T, H, dtype=f_dtype, device=device)
+                d_g = torch.empty(B, U, H, dtype=g_dtype, device=device)
+                dg_part = torch.empty(chunks, B, U, H, dtype=torch.float32, device=device)
+            else:
+                dg_part = None
             if ctx.needs_input_grad[2]:
-                d_weight = dw_part.sum(0)[:VD].to(weight.dtype)
+                d_weight = torch.empty(VD, H, dtype=_sum_dtype(weight.dtype), device=device)
             if want_bias:
-                d_bias = db_part.sum(0)[:VD].to(ctx.bias_dtype)
-        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            want_f, want_g = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-            d_f32 = torch.empty(B, T, H, dtype=torch.float32, device=device) if want_f else None
-            # both wanted (the usual case): one pass over d_hidden forms d f and, per run of frames, a share of d g (runs
-            # of a length that U alone decides: the sums then do not depend on how a batch is split into sub-batches).
-            # A workgroup walks its run frame by frame, a barrier each: shorter runs give more workgroups, longer ones
-            # fewer partial sums to add.  Runs of 16 frames against 32, us: the reduction at B=4, T=190, U=49, H=640
-            # 27 / 48; a step at B=16, T=375, H=640, V=257: U=33 472 / 469, U=64 710 / 703, U=121 1139 / 1138.  Few
-            # utterances gain from 16 at larger U too (B=8, T=250, H=256: U=96 270 / 289, U=121 306 / 331), but their
-            # number must not decide.
-            run = 16 if U <= 64 else 32
-            chunks = (T + run - 1) // run if (want_f and want_g and U <= 256) else 0
-            dg_part = torch.empty(chunks, B, U, H, dtype=torch.float32, device=device) if chunks else None
-            d_g32 = torch.empty(B, U, H, dtype=torch.float32, device=device) if (want_g and not chunks) else None
+                d_bias = torch.empty(VD, dtype=_sum_dtype(ctx.bias_dtype), device=device)
+            with torch.cuda.device(device):
+                status = lib.mi_joint_gradient_sums(
+                    _ptr(d_hidden) if one_pass else None, _ptr(f16), _ptr(g16), _ptr(act_lens), _ptr(label_lens), _ptr(d_f),
+                    _DTYPE_CODE[f_dtype], _ptr(dg_part), chunks, _ptr(d_g), _DTYPE_CODE[g_dtype], _ptr(dw_part), _ptr(db_part),
+                    slices, _ptr(d_weight), _DTYPE_CODE[_sum_dtype(weight.dtype)], _ptr(d_bias),
+                    _DTYPE_CODE[_sum_dtype(ctx.bias_dtype)], ntiles, dropout, seed, act, B, T, U, H, V, D, NB,
+                    _ptr(workspace), workspace.numel(), _stream(device),
+                )  # fmt: skip
+            _native.check_status(status, "fused joint backward")
+            d_weight = None if d_weight is None else d_weight.to(weight.dtype)  # (nothing to do but for odd dtypes)
+            d_bias = None if d_bias is None else d_bias.to(ctx.bias_dtype)
+        if want_h and not one_pass:
+            d_f = torch.empty(B, T, H, dtype=torch.float32, device=device) if want_f else None
+            d_g = torch.empty(B, U, H, dtype=torch.float32, device=device) if want_g else None
             with torch.cuda.device(device):
                 status = lib.mi_joint_reduce_hidden(
-                    _ptr(d_hidden), _ptr(f16), _ptr(g16), _ptr(act_lens), _ptr(label_lens), _ptr(d_f32), _ptr(d_g32),
-                    _ptr(dg_part), chunks, ntiles, dropout, seed, act, B, T, U, H, V, D, NB, _ptr(workspace),
-                    workspace.numel(), _stream(device),
+                    _ptr(d_hidden), _ptr(f16), _ptr(g16), _ptr(act_lens), _ptr(label_lens), _ptr(d_f), _ptr(d_g), None, 0,
+                    ntiles, dropout, seed, act, B, T, U, H, V, D, NB, _ptr(workspace), workspace.numel(), _stream(device),
                 )  # fmt: skip
             _native.check_status(status, "joint_rnnt_loss backward")
-            d_f = None if d_f32 is None else d_f32.to(ctx.in_dtypes[0])
-            if chunks:
-                d_g = dg_part.sum(0).to(ctx.in_dtypes[1])
-            else:
-                d_g = None if d_g32 is None else d_g32.to(ctx.in_dtypes[1])
+        d_f = None if d_f is None else d_f.to(ctx.in_dtypes[0])
+        d_g = None if d_g is None else d_g.to(ctx.in_dtypes[1])
         return d_f, d_g, d_weight, d_bias, None, None, None, None, None, None, None, None, None, None, None, None
 
 
