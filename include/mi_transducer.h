@@ -405,6 +405,27 @@ int mi_transducer_length_maxima(const int64_t* act_lens, const int64_t* label_le
  * captured).  No event, and nothing that was enqueued behind the kernel is waited for. */
 int mi_transducer_wait_lengths(const int64_t* words, void* stream);
 
+/* The forward calls with that check inside: the first kernel of the call leaves the two maxima in length_maxima
+ * (int64[2], device or pinned host memory; NULL: as the calls without) while the rest of it runs, which saves the
+ * launch in front of it.  The caller sets the words and waits for them as above.  A call that returns an error may
+ * leave them unwritten. */
+int mi_rnnt_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                            const int64_t* label_lens, float* costs, int B, int T, int U, int V, int blank,
+                            float fastemit_lambda, int with_betas, void* prefill_grads, int64_t* length_maxima,
+                            void* workspace, size_t workspace_bytes, void* stream);
+
+int mi_tdt_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                           const int64_t* label_lens, float* costs, int B, int T, int U, int V, int D,
+                           const int32_t* durations_host, int blank, float fastemit_lambda, float sigma,
+                           int use_plain_rnnt, int with_betas, void* prefill_grads, int64_t* length_maxima, void* workspace,
+                           size_t workspace_bytes, void* stream);
+
+int mi_multiblank_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                                  const int64_t* label_lens, float* costs, int B, int T, int U, int V, int num_big_blanks,
+                                  const int32_t* big_blank_durations_host, int blank, float fastemit_lambda, float sigma,
+                                  int with_betas, void* prefill_grads, int64_t* length_maxima, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
 /* ---- diagnostics ------------------------------------------------------------------------
  * Everything from here to the end of this header (mi_transducer_profile_*, mi_transducer_describe_plan,
  * mi_transducer_copy_probe, mi_transducer_prefill_record) binds NO interface of the reference: these are aids for

@@ -71,7 +71,7 @@ namespace {
 // ----------------------------------------------------------------------------------------
 extern "C" {
 
-int mi_transducer_abi_version(void) { return 22; }
+int mi_transducer_abi_version(void) { return 23; }
 
 int mi_transducer_workspace_bytes(int B, int T, int U, int D, size_t* out_bytes) {
   Layout L;
@@ -80,17 +80,27 @@ int mi_transducer_workspace_bytes(int B, int T, int U, int D, size_t* out_bytes)
   return MI_TRANSDUCER_SUCCESS;
 }
 
-int mi_rnnt_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
-                    const int64_t* label_lens, float* costs, int B, int T, int U, int V, int blank,
-                    float fastemit_lambda, int with_betas, void* prefill_grads, void* workspace,
-                    size_t workspace_bytes, void* stream) {
+int mi_rnnt_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                            const int64_t* label_lens, float* costs, int B, int T, int U, int V, int blank,
+                            float fastemit_lambda, int with_betas, void* prefill_grads, int64_t* length_maxima,
+                            void* workspace, size_t workspace_bytes, void* stream) {
   Common c;
   if (!costs) return MI_TRANSDUCER_INVALID_VALUE;
   int st = check_common(acts, act_dtype, labels, act_lens, label_lens, B, T, U, V, 0, blank, workspace,
                         workspace_bytes, stream, &c);
   if (st) return st;
+  c.maxima = length_maxima;
   if ((st = run_denom(c))) return st;
   return run_rnnt_lattice(c, costs, fastemit_lambda, with_betas, with_betas ? prefill_grads : nullptr);
+}
+
+int mi_rnnt_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                    const int64_t* label_lens, float* costs, int B, int T, int U, int V, int blank,
+                    float fastemit_lambda, int with_betas, void* prefill_grads, void* workspace,
+                    size_t workspace_bytes, void* stream) {
+  return mi_rnnt_forward_checked(acts, act_dtype, labels, act_lens, label_lens, costs, B, T, U, V, blank,
+                                 fastemit_lambda, with_betas, prefill_grads, nullptr, workspace, workspace_bytes,
+                                 stream);
 }
 
 int mi_rnnt_backward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
@@ -175,10 +185,11 @@ int mi_rnnt_loss_static(const void* acts, int act_dtype, const int64_t* labels, 
                       grad_mul, B, T, U, V, blank, fastemit_lambda, clamp, riders, ws, L.total, stream);
 }
 
-int mi_tdt_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
-                   const int64_t* label_lens, float* costs, int B, int T, int U, int V, int D,
-                   const int32_t* durations_host, int blank, float fastemit_lambda, float sigma, int use_plain_rnnt,
-                   int with_betas, void* prefill_grads, void* workspace, size_t workspace_bytes, void* stream) {
+int mi_tdt_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                           const int64_t* label_lens, float* costs, int B, int T, int U, int V, int D,
+                           const int32_t* durations_host, int blank, float fastemit_lambda, float sigma,
+                           int use_plain_rnnt, int with_betas, void* prefill_grads, int64_t* length_maxima, void* workspace,
+                           size_t workspace_bytes, void* stream) {
   Common c;
   TdtParams prm;
   if (!costs) return MI_TRANSDUCER_INVALID_VALUE;
@@ -188,10 +199,20 @@ int mi_tdt_forward(const void* acts, int act_dtype, const int64_t* labels, const
   st = check_common(acts, act_dtype, labels, act_lens, label_lens, B, T, U, V, D, blank, workspace, workspace_bytes,
                     stream, &c);
   if (st) return st;
+  c.maxima = length_maxima;
   if ((st = run_denom(c))) return st;
   // omega branch (gpu_rnnt.py:607-622): the plain RNNT recursion over the token logits
   if (use_plain_rnnt) return run_rnnt_lattice(c, costs, fastemit_lambda, with_betas, prefill_grads);
   return run_tdt_lattice(c, costs, fastemit_lambda, with_betas, prm, prefill_grads);
+}
+
+int mi_tdt_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                   const int64_t* label_lens, float* costs, int B, int T, int U, int V, int D,
+                   const int32_t* durations_host, int blank, float fastemit_lambda, float sigma, int use_plain_rnnt,
+                   int with_betas, void* prefill_grads, void* workspace, size_t workspace_bytes, void* stream) {
+  return mi_tdt_forward_checked(acts, act_dtype, labels, act_lens, label_lens, costs, B, T, U, V, D, durations_host,
+                                blank, fastemit_lambda, sigma, use_plain_rnnt, with_betas, prefill_grads, nullptr,
+                                workspace, workspace_bytes, stream);
 }
 
 int mi_tdt_backward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
@@ -302,10 +323,11 @@ int mi_tdt_split_loss(const void* label_acts, const void* duration_acts, int act
                                blank, fastemit_lambda, clamp, sigma, use_plain_rnnt, workspace, workspace_bytes, stream);
 }
 
-int mi_multiblank_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
-                          const int64_t* label_lens, float* costs, int B, int T, int U, int V, int num_big_blanks,
-                          const int32_t* big_blank_durations_host, int blank, float fastemit_lambda, float sigma,
-                          int with_betas, void* prefill_grads, void* workspace, size_t workspace_bytes, void* stream) {
+int mi_multiblank_forward_checked(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                                  const int64_t* label_lens, float* costs, int B, int T, int U, int V, int num_big_blanks,
+                                  const int32_t* big_blank_durations_host, int blank, float fastemit_lambda, float sigma,
+                                  int with_betas, void* prefill_grads, int64_t* length_maxima, void* workspace,
+                                  size_t workspace_bytes, void* stream) {
   Common c;
   MbParams prm;
   if (!costs) return MI_TRANSDUCER_INVALID_VALUE;
@@ -315,8 +337,18 @@ int mi_multiblank_forward(const void* acts, int act_dtype, const int64_t* labels
   st = check_common(acts, act_dtype, labels, act_lens, label_lens, B, T, U, V, 0, blank, workspace, workspace_bytes,
                     stream, &c, num_big_blanks);
   if (st) return st;
+  c.maxima = length_maxima;
   if ((st = run_denom(c))) return st;
   return run_multiblank_lattice(c, costs, fastemit_lambda, with_betas, prm, prefill_grads);
+}
+
+int mi_multiblank_forward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
+                          const int64_t* label_lens, float* costs, int B, int T, int U, int V, int num_big_blanks,
+                          const int32_t* big_blank_durations_host, int blank, float fastemit_lambda, float sigma,
+                          int with_betas, void* prefill_grads, void* workspace, size_t workspace_bytes, void* stream) {
+  return mi_multiblank_forward_checked(acts, act_dtype, labels, act_lens, label_lens, costs, B, T, U, V,
+                                       num_big_blanks, big_blank_durations_host, blank, fastemit_lambda, sigma,
+                                       with_betas, prefill_grads, nullptr, workspace, workspace_bytes, stream);
 }
 
 int mi_multiblank_backward(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,

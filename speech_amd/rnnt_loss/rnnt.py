@@ -88,6 +88,12 @@ def new_workspace(acts, num_durations=0):
     return torch.empty(nbytes, dtype=torch.uint8, device=acts.device)
 
 
+def _check_maxima(words):
+    if words is not None and (words.dtype != torch.int64 or words.numel() != 2 or not words.is_contiguous()
+                              or not (words.is_cuda or words.is_pinned())):  # fmt: skip
+        raise ValueError("length_maxima: out must be an int64[2] device or pinned host tensor")
+
+
 def length_maxima(act_lens, label_lens, out=None):
     """int64[2] = (max(act_lens), max(label_lens)), enqueued on the current stream.  `out` may be a
     pinned host tensor: the kernel then writes the two values straight into host memory (pinned
@@ -95,8 +101,7 @@ def length_maxima(act_lens, label_lens, out=None):
     _require_gpu(act_lens, "length_maxima")
     if out is None:
         out = torch.empty(2, dtype=torch.int64, device=act_lens.device)
-    elif out.dtype != torch.int64 or out.numel() != 2 or not (out.is_cuda or out.is_pinned()):
-        raise ValueError("length_maxima: out must be an int64[2] device or pinned host tensor")
+    _check_maxima(out)
     with _on(act_lens.device):
         status = _native.lib().mi_transducer_length_maxima(
             _ptr(act_lens), _ptr(label_lens), act_lens.shape[0], _ptr(out), _stream(act_lens.device)
@@ -110,8 +115,8 @@ LENGTHS_PENDING = -(2**63)
 
 
 def wait_lengths(words, stream):
-    """Return once the kernel of length_maxima(..., out=words), enqueued on `stream`, has written both words (a pinned
-    host tensor that held LENGTHS_PENDING before)."""
+    """Return once the kernel of length_maxima(..., out=words), or of a forward call with maxima=words, enqueued on
+    `stream`, has written both words (a pinned host tensor that held LENGTHS_PENDING before), or `stream` is idle."""
     status = _native.lib().mi_transducer_wait_lengths(_ptr(words), ctypes.c_void_p(stream.cuda_stream))
     _native.check_status(status, "length check")
 
@@ -161,18 +166,21 @@ def tdt_lattice(act_lens, label_lens, costs, B, T, U, durations, fastemit_lambda
 
 
 def rnnt_forward(acts, labels, act_lens, label_lens, costs, blank, fastemit_lambda, with_betas, workspace,
-                 prefill_grads=None):
+                 prefill_grads=None, maxima=None):
     """prefill_grads: the buffer (shape and dtype of acts) that the backward call of this forward call will write the
     gradient into, or None.  While the lattice recursion runs, extra workgroups of its launch zero-fill the padded
-    cells of that buffer as far as they get; rnnt_backward(..., padding_zeroed=2) then skips what they did."""
+    cells of that buffer as far as they get; rnnt_backward(..., padding_zeroed=2) then skips what they did.
+    maxima: int64[2], on the device or in pinned host memory, that receives (max(act_lens), max(label_lens)) from the call's first kernel,
+    as length_maxima(out=maxima) in front of the call would leave them; None: not wanted."""
     _require_gpu(acts, "rnnt_forward")
     B, T, U, V = acts.shape
     _check_prefill(acts, prefill_grads)
+    _check_maxima(maxima)
     with _on(acts.device):
-        status = _native.lib().mi_rnnt_forward(
+        status = _native.lib().mi_rnnt_forward_checked(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, V, int(blank), float(fastemit_lambda), int(bool(with_betas)), _ptr(prefill_grads),
-            _ptr(workspace), workspace.numel(), _stream(acts.device),
+            _ptr(maxima), _ptr(workspace), workspace.numel(), _stream(acts.device),
         )  # fmt: skip
     _native.check_status(status, "Could not calculate forward scores")
 
@@ -197,19 +205,21 @@ def rnnt_backward(
 
 def tdt_forward(
     acts, labels, act_lens, label_lens, costs, blank, durations, fastemit_lambda, sigma, use_plain_rnnt, with_betas,
-    workspace, prefill_grads=None,
+    workspace, prefill_grads=None, maxima=None,
 ):  # fmt: skip
-    """prefill_grads: as for rnnt_forward."""
+    """prefill_grads, maxima: as for rnnt_forward."""
     _require_gpu(acts, "tdt_forward")
     B, T, U, VD = acts.shape
     _check_prefill(acts, prefill_grads)
+    _check_maxima(maxima)
     D = len(durations)
     keep, dur_ptr = _durations_array(durations)
     with _on(acts.device):
-        status = _native.lib().mi_tdt_forward(
+        status = _native.lib().mi_tdt_forward_checked(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, VD - D, D, dur_ptr, int(blank), float(fastemit_lambda), float(sigma), int(bool(use_plain_rnnt)),
-            int(bool(with_betas)), _ptr(prefill_grads), _ptr(workspace), workspace.numel(), _stream(acts.device),
+            int(bool(with_betas)), _ptr(prefill_grads), _ptr(maxima), _ptr(workspace), workspace.numel(),
+            _stream(acts.device),
         )  # fmt: skip
     del keep
     _native.check_status(status, "Could not calculate forward scores")
@@ -236,18 +246,20 @@ def tdt_backward(
 
 def multiblank_forward(
     acts, labels, act_lens, label_lens, costs, blank, big_blank_durations, fastemit_lambda, sigma, with_betas, workspace,
-    prefill_grads=None,
+    prefill_grads=None, maxima=None,
 ):  # fmt: skip
-    """prefill_grads: as for rnnt_forward."""
+    """prefill_grads, maxima: as for rnnt_forward."""
     _require_gpu(acts, "multiblank_forward")
     B, T, U, V = acts.shape
     _check_prefill(acts, prefill_grads)
+    _check_maxima(maxima)
     keep, dur_ptr = _durations_array(big_blank_durations)
     with _on(acts.device):
-        status = _native.lib().mi_multiblank_forward(
+        status = _native.lib().mi_multiblank_forward_checked(
             _ptr(acts), _dtype_code(acts), _labels_ptr(labels), _ptr(act_lens), _ptr(label_lens), _ptr(costs),
             B, T, U, V, len(big_blank_durations), dur_ptr, int(blank), float(fastemit_lambda), float(sigma),
-            int(bool(with_betas)), _ptr(prefill_grads), _ptr(workspace), workspace.numel(), _stream(acts.device),
+            int(bool(with_betas)), _ptr(prefill_grads), _ptr(maxima), _ptr(workspace), workspace.numel(),
+            _stream(acts.device),
         )  # fmt: skip
     del keep
     _native.check_status(status, "Could not calculate forward scores")

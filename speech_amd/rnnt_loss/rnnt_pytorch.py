@@ -151,29 +151,33 @@ _STRICT_LENGTH_CHECK = os.environ.get("MI_TRANSDUCER_STRICT_LENGTH_CHECK", "") =
 
 class _PendingLengthCheck:
     """The T == max(act_lens), U == max(label_lens)+1 test of certify_inputs, split in two
-    so that the read-back of the maxima overlaps kernels enqueued in between."""
+    so that the read-back of the maxima overlaps kernels enqueued in between.  forward_follows: the caller hands
+    `maxima` (None where there is nothing to fill) to the forward call as maxima=, whose first kernel fills it."""
 
-    def __init__(self, log_probs, lengths, label_lengths):
+    def __init__(self, log_probs, lengths, label_lengths, forward_follows=False):
         self.T, self.U = log_probs.shape[1:3]
         self.padded_T = _caller_mode.padded_time_axis
         self.key = (lengths._version, label_lengths._version, self.T, self.U, self.padded_T)
         self.tensors = (lengths, label_lengths)
-        self.host = self.stream = None
+        self.host = self.stream = self.maxima = None
         seen = _validated.entry
         if (not _STRICT_LENGTH_CHECK and seen is not None and seen[0]() is lengths and seen[1]() is label_lengths
                 and seen[2] == self.key):
             return  # these very tensors, unmodified, passed against this shape
         if lengths.is_cuda:
-            # One small kernel in front of the first kernel of the loss, on the same stream, writes the two maxima into
-            # pinned host memory; finish() looks at the words until they are there.  (On a stream of its own, behind
-            # an event, the kernel overlaps pass 1, but the event leaves a gap in front of pass 1 that is longer than
-            # the kernel, and stream, events and record_stream cost the host 40 to 60 us a call.  Step at B=4, T=50,
-            # U=21, V=129 233 -> 166 us, forward alone at B=8, T=187, U=46, V=1025 85 -> 47 us.)
+            # The first kernel of the loss (or one small kernel) writes the two maxima into pinned host memory; finish()
+            # looks at the words until they are there.  (A small kernel in front of every loss, on the same stream: a
+            # launch and a gap more, 2 us on the device and 6 on the host.  On a stream of its own, behind an event, it overlaps pass 1, but the event
+            # leaves a gap in front of pass 1 that is longer than the kernel, and stream, events and record_stream cost
+            # the host 40 to 60 us a call.)
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("the shape check of new length tensors reads the lengths back: it cannot be captured")
             self.host, words = _length_words.get()
             words[0] = words[1] = rnnt.LENGTHS_PENDING
-            rnnt.length_maxima(lengths, label_lengths, out=self.host)
+            if forward_follows:
+                self.maxima = self.host
+            else:
+                rnnt.length_maxima(lengths, label_lengths, out=self.host)
             self.stream = torch.cuda.current_stream(lengths.device)
         else:
             self.host = torch.stack([torch.max(lengths), torch.max(label_lengths)])
@@ -291,7 +295,7 @@ class _RNNTNumba(Function):
                 ctx.save_for_backward(acts, labels, act_lens, label_lens, workspace)
                 ctx.params = (blank, reduction, fastemit_lambda, clamp)
             return costs
-        pending = _PendingLengthCheck(acts, act_lens, label_lens)
+        pending = _PendingLengthCheck(acts, act_lens, label_lens, forward_follows=True)
         try:
             need_grad = ctx.needs_input_grad[0]
             batch = acts.size(0)
@@ -299,7 +303,7 @@ class _RNNTNumba(Function):
             workspace = rnnt.new_workspace(acts)
             ctx.prefilled = grads_like(acts) if need_grad and _prefill_wanted(acts) else None
             rnnt.rnnt_forward(acts, labels, act_lens, label_lens, costs, blank, fastemit_lambda, need_grad, workspace,
-                              ctx.prefilled)
+                              ctx.prefilled, pending.maxima)
         except BaseException:
             pending.drain()  # the pinned buffer must outlive the kernel that writes into it
             raise
@@ -349,7 +353,7 @@ class _TDTNumba(Function):
         durations = [int(d) for d in durations]
         if acts.shape[-1] <= len(durations):
             raise ValueError("acts must hold the token logits followed by one logit per duration")
-        pending = _PendingLengthCheck(acts, act_lens, label_lens)
+        pending = _PendingLengthCheck(acts, act_lens, label_lens, forward_follows=True)
         try:
             need_grad = ctx.needs_input_grad[0]
             batch = acts.size(0)
@@ -360,7 +364,7 @@ class _TDTNumba(Function):
             ctx.prefilled = grads_like(acts) if need_grad and _prefill_wanted(acts) else None
             rnnt.tdt_forward(
                 acts, labels, act_lens, label_lens, costs, blank, durations, fastemit_lambda, sigma, use_plain_rnnt,
-                need_grad, workspace, ctx.prefilled,
+                need_grad, workspace, ctx.prefilled, pending.maxima,
             )  # fmt: skip
         except BaseException:
             pending.drain()  # the pinned buffer must outlive the kernel that writes into it
@@ -406,7 +410,7 @@ class _MultiblankRNNTNumba(Function):
         durations = [int(d) for d in big_blank_durations]
         if blank - len(durations) < 0 or blank >= acts.shape[-1]:
             raise ValueError("the big blanks sit at blank-1-i: blank must leave room for them below it")
-        pending = _PendingLengthCheck(acts, act_lens, label_lens)
+        pending = _PendingLengthCheck(acts, act_lens, label_lens, forward_follows=True)
         try:
             need_grad = ctx.needs_input_grad[0]
             batch = acts.size(0)
@@ -415,7 +419,7 @@ class _MultiblankRNNTNumba(Function):
             ctx.prefilled = grads_like(acts) if need_grad and _prefill_wanted(acts) else None
             rnnt.multiblank_forward(
                 acts, labels, act_lens, label_lens, costs, blank, durations, fastemit_lambda, sigma, need_grad, workspace,
-                ctx.prefilled,
+                ctx.prefilled, pending.maxima,
             )  # fmt: skip
         except BaseException:
             pending.drain()  # the pinned buffer must outlive the kernel that writes into it
