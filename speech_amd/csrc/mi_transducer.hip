@@ -115,8 +115,9 @@ int mi_rnnt_backward(const void* acts, int act_dtype, const int64_t* labels, con
   if (st) return st;
   const ScaleArg sc = {grad_scale, grad_scale_stride, grad_mul};
   const bool fused = rnnt_rows_fused(c, grads);
-  if (!fused && (st = run_rnnt_cells(c, sc, fastemit_lambda, clamp))) return st;
-  return run_grad_stream(c, grads, padding_flags(padding_zeroed), fused, sc, fastemit_lambda, clamp);
+  const bool short_records = !fused && rnnt_short_records(c, grads);
+  if (!fused && (st = run_rnnt_cells(c, sc, fastemit_lambda, clamp, short_records))) return st;
+  return run_grad_stream(c, grads, padding_flags(padding_zeroed), fused, sc, fastemit_lambda, clamp, short_records);
 }
 
 int mi_rnnt_loss(const void* acts, int act_dtype, const int64_t* labels, const int64_t* act_lens,
