@@ -33,7 +33,7 @@ import random
 import torch
 
 from speech_amd import _native
-from speech_amd.rnnt_loss.rnnt import _DTYPE_CODE, _durations_array, _labels_ptr, _ptr, _require_gpu, _stream
+from speech_amd.rnnt_loss.rnnt import _DTYPE_CODE, _durations_array, _labels_ptr, _on, _ptr, _require_gpu, _stream
 
 __all__ = ["joint_rnnt_forward", "joint_rnnt_loss", "joint_tdt_forward", "joint_tdt_loss", "joint_multiblank_forward",
            "joint_multiblank_loss", "joint_dropout_mask", "JointRNNTLoss"]  # fmt: skip
@@ -102,7 +102,7 @@ def _draw_seed(dropout, seed):
 def joint_dropout_mask(B, T, U, H, dropout, seed, device):
     """The keep mask [B,T,U,H] (bool) the kernels derive from (seed, cell, hidden unit), for tests."""
     mask = torch.empty(B, T, U, H, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         status = _native.lib().mi_joint_dropout_mask(_ptr(mask), float(dropout), int(seed), B, T, U, H, _stream(device))
     _native.check_status(status, "joint_dropout_mask")
     return mask.bool()
@@ -131,7 +131,7 @@ def _forward(f16, g16, weight, bias, labels, act_lens, label_lens, blank, fastem
     tiles = torch.empty(1, dtype=torch.int32, device=device)
     wcode = _native.DTYPE_F32 if wdtype == torch.float32 else _native.DTYPE_BF16
     keep_args = (None, None, 0) if saved is None else (_ptr(saved[0]), _ptr(saved[1]), saved[0].shape[0] // 128)
-    with torch.cuda.device(device):
+    with _on(device):
         if D:
             keep, dur_ptr = _durations_array(durations)
             status = _native.lib().mi_joint_tdt_forward(
@@ -264,7 +264,7 @@ class JointRNNTLoss(torch.autograd.Function):
         d_weight = d_bias = d_f = d_g = None
         if want_w or want_h:
             outs = (_ptr(logits16), _ptr(acts), _ptr(d_hidden), _ptr(dw_part), _ptr(db_part), slices, ntiles)
-            with torch.cuda.device(device):
+            with _on(device):
                 if D:
                     keep, dur_ptr = _durations_array(durations)
                     status = lib.mi_joint_tdt_backward(
@@ -311,7 +311,7 @@ class JointRNNTLoss(torch.autograd.Function):
                 d_weight = torch.empty(VD, H, dtype=_sum_dtype(weight.dtype), device=device)
             if want_bias:
                 d_bias = torch.empty(VD, dtype=_sum_dtype(ctx.bias_dtype), device=device)
-            with torch.cuda.device(device):
+            with _on(device):
                 status = lib.mi_joint_gradient_sums(
                     _ptr(d_hidden) if one_pass else None, _ptr(f16), _ptr(g16), _ptr(act_lens), _ptr(label_lens), _ptr(d_f),
                     _DTYPE_CODE[f_dtype], _ptr(dg_part), chunks, _ptr(d_g), _DTYPE_CODE[g_dtype], _ptr(dw_part), _ptr(db_part),
@@ -325,7 +325,7 @@ class JointRNNTLoss(torch.autograd.Function):
         if want_h and not one_pass:
             d_f = torch.empty(B, T, H, dtype=torch.float32, device=device) if want_f else None
             d_g = torch.empty(B, U, H, dtype=torch.float32, device=device) if want_g else None
-            with torch.cuda.device(device):
+            with _on(device):
                 status = lib.mi_joint_reduce_hidden(
                     _ptr(d_hidden), _ptr(f16), _ptr(g16), _ptr(act_lens), _ptr(label_lens), _ptr(d_f), _ptr(d_g), None, 0,
                     ntiles, dropout, seed, act, B, T, U, H, V, D, NB, _ptr(workspace), workspace.numel(), _stream(device),

@@ -47,11 +47,14 @@ def _require_gpu(t, what):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()  # (an integer: the signatures make a pointer of it)
 
 
 def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # (the handle alone; torch.cuda.current_stream builds a Stream object around it, 4 us a call)
+    if isinstance(device, torch.device) and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 _NO_SWITCH = contextlib.nullcontext()
@@ -114,10 +117,10 @@ def length_maxima(act_lens, label_lens, out=None):
 LENGTHS_PENDING = -(2**63)
 
 
-def wait_lengths(words, stream):
+def wait_lengths(words, stream):  # (stream: a torch.cuda.Stream or its handle)
     """Return once the kernel of length_maxima(..., out=words), or of a forward call with maxima=words, enqueued on
     `stream`, has written both words (a pinned host tensor that held LENGTHS_PENDING before), or `stream` is idle."""
-    status = _native.lib().mi_transducer_wait_lengths(_ptr(words), ctypes.c_void_p(stream.cuda_stream))
+    status = _native.lib().mi_transducer_wait_lengths(_ptr(words), getattr(stream, "cuda_stream", stream))
     _native.check_status(status, "length check")
 
 

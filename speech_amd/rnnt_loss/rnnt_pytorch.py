@@ -21,7 +21,7 @@ What is done differently underneath:
     `acts`, as the reference does (which computes the gradient there): the lattice launch
     zero-fills its padded cells while it runs.  That tensor is held until backward runs or
     the graph is dropped; MI_TRANSDUCER_PREFILL=0 in the environment restores the small footprint.
-  * the shape-vs-lengths check has one small kernel write both maxima into host memory and
+  * the shape-vs-lengths check has the first kernel leave both maxima in host memory and
     looks at them once the forward kernels are enqueued, instead of two blocking torch.max calls.
 """
 
@@ -159,7 +159,7 @@ class _PendingLengthCheck:
         self.padded_T = _caller_mode.padded_time_axis
         self.key = (lengths._version, label_lengths._version, self.T, self.U, self.padded_T)
         self.tensors = (lengths, label_lengths)
-        self.host = self.stream = self.maxima = None
+        self.host = self.words = self.stream = self.maxima = None
         seen = _validated.entry
         if (not _STRICT_LENGTH_CHECK and seen is not None and seen[0]() is lengths and seen[1]() is label_lengths
                 and seen[2] == self.key):
@@ -172,13 +172,13 @@ class _PendingLengthCheck:
             # the host 40 to 60 us a call.)
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError("the shape check of new length tensors reads the lengths back: it cannot be captured")
-            self.host, words = _length_words.get()
-            words[0] = words[1] = rnnt.LENGTHS_PENDING
+            self.host, self.words = _length_words.get()
+            self.words[0] = self.words[1] = rnnt.LENGTHS_PENDING
             if forward_follows:
                 self.maxima = self.host
             else:
                 rnnt.length_maxima(lengths, label_lengths, out=self.host)
-            self.stream = torch.cuda.current_stream(lengths.device)
+            self.stream = rnnt._stream(lengths.device)
         else:
             self.host = torch.stack([torch.max(lengths), torch.max(label_lengths)])
 
@@ -193,7 +193,7 @@ class _PendingLengthCheck:
         if self.host is None:
             return
         self.drain()
-        max_T, max_U = int(self.host[0]), int(self.host[1])
+        max_T, max_U = (int(w) for w in (self.host if self.words is None else self.words))
         if self.T < max_T if self.padded_T else self.T != max_T:
             raise ValueError(f"Input length mismatch! Given T: {self.T}, Expected max T from input lengths: {max_T}")
         if self.U != max_U + 1:
