@@ -123,3 +123,26 @@ def test_plan_lines():
         assert (tdt == "tdt_lattice_pair_kernel<D=5>") == scaled, (U, longest, tdt)
         mb = _native.describe_plan(0, 4, 100, U, 68, max_duration=longest, num_big_blanks=3)["lattice"]
         assert (mb == "multiblank_lattice_kernel<NBC=4>") == scaled, (U, longest, mb)
+
+
+@gpu
+@pytest.mark.parametrize("sigma", [0.7, 1.5, -0.8])
+@pytest.mark.parametrize("value", [-1.0e10, -1.0e30, float(np.finfo(np.float32).min)])
+@pytest.mark.parametrize("kind,steps,column", [
+    ("tdt", [0, 1, 2, 3, 4], "blank"), ("tdt", [0, 1, 2, 3, 4], "label"), ("tdt", [0, 1, 2, 3, 4], "step"),
+    ("tdt", [0, 1, 2, 6], "step"), ("multiblank", [2, 4, 8], "blank"), ("multiblank", [2, 4, 8], "label"),
+    ("multiblank", [2, 4], "step")])  # fmt: skip
+def test_masked_arcs_whatever_sigma(kind, steps, column, value, sigma):
+    """An arc that is masked out, far below the range of a float exponent: in all cells for a duration (or big blank), in one for
+    a token, of an utterance without labels, one with some and one with all of them.  Every utterance keeps a path without it."""
+    acts, labels, _, _ = draw(17, kind, 3, 9, 5, steps)
+    blank = acts.shape[-1] - 1 - (len(steps) if kind == "tdt" else 0)
+    acts = acts.astype(np.float32)
+    if column == "step":
+        acts[..., acts.shape[-1] - 1 if kind == "tdt" else blank - 1] = value
+    elif column == "blank":
+        acts[:, 3, :, blank] = value
+    else:
+        for b in range(3):
+            acts[b, 3, 1, labels[b, 1]] = value
+    check(kind, acts, labels, [9, 9, 8], [0, 2, 4], steps, sigma=sigma)
