@@ -146,3 +146,28 @@ def test_masked_arcs_whatever_sigma(kind, steps, column, value, sigma):
         for b in range(3):
             acts[b, 3, 1, labels[b, 1]] = value
     check(kind, acts, labels, [9, 9, 8], [0, 2, 4], steps, sigma=sigma)
+
+
+def steep(kind, steps, level, T, U, B=2, seed=0, jitter=0.0):
+    """Logits whose arcs all have log-probs of `level`, beside one likely token that is no label and, for TDT, a likely duration of
+    0: long steps and runs of short ones reach the same cells with hundreds of bits between them on the way."""
+    rng = np.random.RandomState(seed)
+    tokens = 6
+    acts = rng.randn(B, T, U, tokens + 1 + len(steps)) * jitter
+    labels = rng.randint(0, tokens - 1, size=(B, U - 1))  # (token 5 is never a label)
+    if kind == "tdt":
+        acts[..., 5] -= level  # blank and labels at `level`
+        acts[..., tokens + 1] -= level  # duration 0: of no use to a blank
+    else:
+        acts[..., 5] -= level
+    return acts, labels
+
+
+@gpu
+@pytest.mark.parametrize("level", [-40.0, -50.0, -55.0, -59.0])
+@pytest.mark.parametrize("kind,steps,T,U", [("tdt", [0, 1, 8], 15, 1), ("tdt", [0, 1, 8], 40, 1), ("tdt", [0, 1, 8], 31, 9), ("tdt", [0, 1, 2, 8], 30, 4), ("tdt", [0, 1, 6], 25, 7),
+                                            ("tdt", [0, 1, 4], 29, 12), ("tdt", [0, 1, 8], 24, 70), ("multiblank", [8], 33, 5), ("multiblank", [2, 8], 24, 70)])  # fmt: skip
+def test_long_steps_beside_runs_of_short_ones(kind, steps, T, U, level):
+    """Costs of about 100 * level, each log-prob rounded by 2^-24 of its size: up to (T + U) * 60 * 2 * 2^-24 in an exponent."""
+    acts, labels = steep(kind, steps, level, T, U)
+    check(kind, acts, labels, [T, T - 2], [U - 1, U // 2], steps, sigma=0.05, lam=0.0, grad_atol=(T + U) * 120 * 2.0**-24)

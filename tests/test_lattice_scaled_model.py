@@ -1,0 +1,267 @@
+"""The recursion of TDT and multi-blank lattices on probabilities (mi_scaled.inc), restated in numpy with its columns' exponents and
+the guard that sends an utterance to the recursion on logarithms.  Held against the recursion in 64-bit logarithms on arcs up
+to the edge of the guard's range, in the patterns that pull the values of a column apart: whatever the guard lets pass is
+right, and it lets ordinary lattices pass.  The GPU tests of the kernels are in test_gpu_lattice_scaled.py."""
+
+import os
+import re
+
+import numpy as np
+import pytest
+
+SOURCE = os.path.join(os.path.dirname(__file__), "..", "speech_amd", "csrc", "mi_scaled.inc")
+
+
+def constant(name):
+    with open(SOURCE) as file:
+        return eval(re.search(rf"constexpr int {name} = ([^;]+);|, {name} = (-?\d+);", file.read()).group(1))
+
+
+SLOPE, LAG, MASSLESS = constant("kScaledSlope"), constant("kScaledLag"), constant("kScaledMassless")
+
+
+def high_word(x):
+    return np.ascontiguousarray(x).view(np.int64) >> 32
+
+
+def scale(x, bits):
+    return np.ldexp(x, np.clip(bits, -5000, 5000).astype(np.int32))
+
+
+def recursion(tdt, longest, beta, factors, diagonals, steps, batch):
+    """factors [n, steps, positions, NV] of n lattices: what the helpers leave.  Returns the cells' mantissas and the columns'
+    exponents by step and position.  longest: MAXD, batch: P."""
+    n, _, columns, _ = factors.shape
+    every = 4 if tdt else 8
+    turn = max(longest, every, batch)
+    total = (steps + turn - 1) // turn * turn
+    values, exponents = np.zeros((n, total, columns)), np.zeros((n, total, columns), dtype=np.int64)
+    edge, edge_exponent = np.zeros((n, total)), np.zeros((n, total), dtype=np.int64)
+    for g0 in range(0, columns, 64):
+        width = min(64, columns - g0)
+        lane = np.arange(width)
+        own, passed = np.zeros((longest, n, width)), np.zeros((longest if tdt else 1, n, width))  # S and N
+        send = np.zeros((n, width))
+        if g0 == 0:
+            own[longest - 1 if beta else 0][:, 0] = 1.0
+        e, shift_in = np.zeros((n, width), dtype=np.int64), np.zeros((n, width), dtype=np.int64)
+        next_edge, next_exponent = np.zeros((n, total)), np.zeros((n, total), dtype=np.int64)
+        for i in range(total):
+            if i % every == 0:
+                top = np.maximum.reduce([high_word(x) for x in [send, *own, *(passed if tdt else [])]])
+                fed = np.full(n, 2 * MASSLESS)
+                if g0:  # what comes in at the steps of this batch until the next time, by the exponents of the steps before
+                    for s in range(i, min(i + every, (i // batch + 1) * batch)):
+                        fed = np.maximum(fed, edge_exponent[:, s - 1] if s else 0)
+                had = np.where(top > 0, e + (top >> 20) - 1023, MASSLESS)
+                below = np.concatenate([fed[:, None], had[:, :-1]], axis=1)
+                steep = (had < below - SLOPE).any(axis=1)
+                raised = np.maximum(np.maximum.accumulate(had + SLOPE * lane, axis=1), fed[:, None] - SLOPE) - SLOPE * lane
+                now = np.where(steep[:, None], raised, had)
+                own, send = scale(own, e - now), scale(send, e - now)
+                if tdt:
+                    passed = scale(passed, e - now)
+                e = now
+                shift_in = np.minimum(np.concatenate([e[:, :1], e[:, :-1]], axis=1) - e, SLOPE)
+            exponents[:, i, g0 : g0 + width] = e
+            fill = np.zeros(n)
+            if g0 and i:
+                fill = scale(edge[:, i - 1], np.minimum(edge_exponent[:, i - 1] - e[:, 0], SLOPE))
+            come = scale(np.concatenate([fill[:, None], send[:, :-1]], axis=1), shift_in)
+            f = factors[:, i, g0 : g0 + width].transpose(2, 0, 1) if i < steps else np.zeros((factors.shape[3], n, width))
+            if not beta:
+                if tdt and i == diagonals:
+                    come = np.zeros_like(come)
+                a = own[0] + come
+                b, ways = (a * f[0], f[2:]) if tdt else (a, f)
+                own = np.concatenate([own[1:], np.zeros((1, n, width))]) + b * ways[1:]
+                if tdt:
+                    label = a * f[1]
+                    send = label * ways[0] + passed[0]
+                    passed = np.concatenate([passed[1:], np.zeros((1, n, width))]) + label * ways[1:]
+                else:
+                    send = a * f[0]
+                handed = send
+            else:  # own[-1] is one step old
+                if tdt:
+                    a = (come * f[2] + (passed[::-1] * f[3:]).sum(0)) * f[1] + (own[::-1] * f[3:]).sum(0) * f[0]
+                    passed = np.concatenate([passed[1:], come[None]])
+                else:
+                    a = come * f[0] + (own[::-1] * f[1:]).sum(0)
+                own = np.concatenate([own[1:], a[None]])
+                send = handed = a
+            values[:, i, g0 : g0 + width] = a
+            next_edge[:, i], next_exponent[:, i] = handed[:, -1], e[:, -1]
+        edge, edge_exponent = next_edge, next_exponent
+    return values, exponents
+
+
+def guard(tdt, durations, longest, values, exponents, end, T, batch):
+    """Whether a lattice runs again on logarithms, as the helpers find out batch by batch."""
+    n, total, columns = values.shape
+    i, pos = np.arange(total)[:, None], np.arange(columns)[None]
+    valid = (i >= pos) & (i - pos < T)
+    mass = high_word(values) > 0
+    bad = ~(np.isfinite(end) & (end > 0))
+    bad |= (valid & (i >= (2 * pos if tdt and 0 not in durations else pos)) & ~mass).any((1, 2))
+    x = np.where(mass & valid, np.frexp(values)[1] + exponents, 1 << 40)
+    low = x.reshape(n, -1, batch, columns).min(2)
+    high = exponents.reshape(n, -1, batch, columns).max(2)
+    for q in range(low.shape[1]):
+        for w in range(min(q, (batch - 1 + longest) // batch) + 1):
+            bad |= ((low[:, q - w] < high[:, q] - LAG) | (low[:, q] < high[:, q - w] - LAG)).any(1)
+    return bad
+
+
+def reference(tdt, durations, blank, label, ways):
+    """alpha [n, T, U], beta and the total in logarithms.  blank, label [n, T, U], ways [n, T, U, D] (multi-blank: its blank arcs)."""
+    n, T, U = label.shape
+    none, far = -np.inf, T + max(durations)
+    alpha, beta, total = np.full((n, far, U), none), np.full((n, far, U), none), np.full(n, none)
+    alpha[:, 0, 0] = 0.0
+    for t in range(T):
+        for u in range(U):
+            for k, d in enumerate(durations):
+                way = alpha[:, t, u] + ways[:, t, u, k]
+                if d > 0 and (t + d < T or (t + d == T and u == U - 1)):
+                    step = way + (blank[:, t, u] if tdt else 0.0)
+                    if t + d < T:
+                        alpha[:, t + d, u] = np.logaddexp(alpha[:, t + d, u], step)
+                    else:
+                        total = np.logaddexp(total, step)
+                if tdt and u + 1 < U and t + d < T:
+                    alpha[:, t + d, u + 1] = np.logaddexp(alpha[:, t + d, u + 1], way + label[:, t, u])
+            if not tdt and u + 1 < U:
+                alpha[:, t, u + 1] = np.logaddexp(alpha[:, t, u + 1], alpha[:, t, u] + label[:, t, u])
+    for t in reversed(range(T)):
+        for u in reversed(range(U)):
+            x = np.full(n, none)
+            for k, d in enumerate(durations):
+                if d > 0 and (t + d < T or (t + d == T and u == U - 1)):
+                    after = beta[:, t + d, u] if t + d < T else 0.0
+                    x = np.logaddexp(x, after + ways[:, t, u, k] + (blank[:, t, u] if tdt else 0.0))
+                if tdt and u + 1 < U and t + d < T:
+                    x = np.logaddexp(x, beta[:, t + d, u + 1] + ways[:, t, u, k] + label[:, t, u])
+            if not tdt and u + 1 < U:
+                x = np.logaddexp(x, beta[:, t, u + 1] + label[:, t, u])
+            beta[:, t, u] = x
+    return alpha[:, :T], beta[:, :T], total
+
+
+def compare(tdt, durations, blank, label, ways, batch=None):
+    """Per lattice and direction: the guard's verdict and the largest error of a cell's posterior (the other direction exact)
+    or of the likelihood."""
+    n, T, U = label.shape
+    longest = 4 if max(durations) <= 4 else 8
+    batch = batch or (8 if U <= 64 * (2 if longest == 4 else 1) else 4)
+    diagonals = T + U - 1
+    exact = reference(tdt, durations, blank, label, ways)
+    verdicts, errors = [], []
+    for beta in (False, True):
+        steps = diagonals + (not beta)
+        factors = np.zeros((n, steps, U, (3 if tdt else 1) + longest))
+        i, pos = np.meshgrid(np.arange(steps), np.arange(U), indexing="ij")
+        u = U - 1 - pos if beta else pos
+        t = (diagonals - 1 - i if beta else i) - u
+        valid = ((t >= 0) & (t < T))[None, :, :, None]
+        t = np.clip(t, 0, T - 1)
+        tokens = np.exp(np.stack([blank[:, t, u], label[:, t, u]], -1)) if tdt else np.exp(label[:, t, u])[..., None]
+        factors[..., : tokens.shape[-1]] = np.where(valid, tokens, 0.0)
+        for k, d in enumerate(durations):
+            factors[..., d + (2 if tdt else 0)] = np.where(valid[..., 0], np.exp(ways[:, t, u, k]), 1.0 if tdt else 0.0)
+        values, exponents = recursion(tdt, longest, beta, factors, diagonals, steps, batch)
+        end = values[:, steps - 1, U - 1]
+        verdicts.append(guard(tdt, durations, longest, values, exponents, end, T, batch))
+        t, u = np.meshgrid(np.arange(T), np.arange(U), indexing="ij")
+        at = (diagonals - 1 - t - u, U - 1 - u) if beta else (t + u, u)
+        mantissa, exponent = np.frexp(values[:, at[0], at[1]])
+        log = (np.log2(mantissa) + exponent + exponents[:, at[0], at[1]]) * np.log(2)
+        total = exact[2][:, None, None]
+        posterior = np.exp(exact[0] + exact[1] - total)
+        error = np.abs(np.exp(log + exact[0 if beta else 1] - total) - posterior)
+        mantissa, exponent = np.frexp(end)
+        end_log = (np.log2(mantissa) + exponent + exponents[:, steps - 1, U - 1]) * np.log(2)
+        error = np.maximum(np.nan_to_num(error, nan=np.inf).max((1, 2)), np.abs(np.expm1(end_log - exact[2])))
+        errors.append(np.nan_to_num(error, nan=np.inf))
+    possible = np.isfinite(exact[2])  # (without an alignment there is nothing to compare)
+    return np.array(verdicts)[:, possible], np.array(errors)[:, possible]
+
+
+# What a pattern varies over (lattice only, cells, columns, frames, quarters of the lattice), each arc either dear or cheap
+def arcs(rng, pattern, n, T, U, dear=-59.9):
+    t, u = np.arange(T)[None, :, None], np.arange(U)[None, None]
+    if pattern == "lattice":
+        x = np.where(rng.rand(n, 1, 1) < 0.6, dear * rng.rand(n, 1, 1), -0.1)
+    elif pattern == "cells":
+        x = np.where(rng.rand(n, T, U) < rng.rand(n, 1, 1), dear, -0.5)
+    elif pattern == "columns":
+        x = np.where(rng.rand(n, 1, U) < 0.5, dear * rng.rand(n, 1, U), -0.1)
+    elif pattern == "frames":
+        x = np.where(rng.rand(n, T, 1) < 0.5, dear * rng.rand(n, T, 1), -0.1)
+    else:
+        quarter = 2 * (t >= rng.randint(0, T, size=(n, 1, 1))) + (u >= rng.randint(0, U, size=(n, 1, 1)))
+        x = np.where(rng.rand(n, 4) < 0.5, dear, -0.1)[np.arange(n)[:, None, None], quarter]
+    return np.broadcast_to(x, (n, T, U))
+
+
+TDT_SETS = [[0, 1, 2, 3, 4], [0, 1, 4], [1, 4], [0, 1, 8], [1, 8], [0, 1, 2, 3, 4, 5, 6, 7, 8], [0, 1, 6], [0, 1]]
+BLANK_SETS = [[1, 2], [1, 4], [1, 2, 4, 8], [1, 8], [1, 3, 5, 7]]  # (the standard blank's 1 among them)
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("pattern", ["lattice", "cells", "columns", "frames", "quarters"])
+@pytest.mark.parametrize("tdt,durations", [(True, d) for d in TDT_SETS] + [(False, d) for d in BLANK_SETS])
+def test_what_the_guard_passes_is_right(pattern, tdt, durations):
+    """A value's relative error is some 2^-53 a step, and the logarithms' own rounding up to (T + U) * 120 * 2^-53 = 2e-12."""
+    rng = np.random.RandomState(len(pattern) + 100 * sum(durations) + tdt)
+    for T, U in [(25, 1), (9, 2), (17, 5), (30, 9), (8, 40), (5, 70)]:
+        blank, label = arcs(rng, pattern, 10, T, U), arcs(rng, pattern, 10, T, U)
+        ways = np.stack([arcs(rng, pattern, 10, T, U) for _ in durations], -1)
+        verdicts, errors = compare(tdt, durations, blank, label, ways)
+        assert not (errors[~verdicts] > 1e-10).any(), (T, U, errors[~verdicts].max())
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("U", [1, 2, 5, 70])
+@pytest.mark.parametrize("tdt,durations", [(True, d) for d in TDT_SETS] + [(False, d) for d in BLANK_SETS])
+def test_every_arc_at_one_level(tdt, durations, U):
+    """Runs of short steps beside long ones, and columns that cost 174 bits each.  (The random patterns rarely need the distances
+    that the guard watches, cells without mass tell nearly all; of these, TDT with [0, 1, 8] and 70 columns with any set do.)"""
+    levels = np.linspace(-59.9, -30.0, 8)[:, None, None]
+    for T in range(2, 34, 1 if U < 5 else 3) if U < 70 else (3, 4, 5, 6):
+        dear = np.broadcast_to(levels, (8, T, U))
+        verdicts, errors = compare(tdt, durations, dear, dear, np.stack([dear] * len(durations), -1))
+        assert not (errors[~verdicts] > 1e-10).any(), (T, errors[~verdicts].max())
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+def test_a_long_step_beside_seven_short_ones():
+    """Seven blanks of duration 1 and a step of 8 from there are as likely as a step of 8 and seven blanks behind it: alpha's total
+    lacks the one and beta's first cell all of it, unless the guard finds them."""
+    dear = np.full((1, 15, 1), -55.0)
+    verdicts, errors = compare(True, [0, 1, 8], dear, dear, np.stack([dear] * 3, -1))
+    assert verdicts.all() and (errors > 0.1).all()
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("tdt,durations", [(True, [0, 1, 2, 3, 4]), (True, list(range(9))), (True, [1, 2, 3, 4]), (False, [1, 2, 4, 8])])
+@pytest.mark.parametrize("spread", [1.0, 3.0, 6.0])
+def test_ordinary_lattices_pass(tdt, durations, spread):
+    rng = np.random.RandomState(int(spread))
+
+    def log_softmax(x):
+        return x - np.log(np.exp(x).sum(-1, keepdims=True))
+
+    x = log_softmax(rng.randn(4, 60, 20, 64) * spread)
+    ways = log_softmax(rng.randn(4, 60, 20, len(durations)) * spread) if tdt else x[..., [0, 2, 3, 4]]
+    verdicts, errors = compare(tdt, durations, x[..., 0], x[..., 1], ways)
+    assert not verdicts.any() and errors.max() < 1e-9
+
+
+def test_the_bounds_fit_a_double():
+    """A cell LAG bits down pushes through two arcs at the lower bound, with the rounding of an exponent each: normal still.  Upwards,
+    four steps (TDT: two arcs each) or eight of the largest factors and slopes stay finite."""
+    with open(SOURCE) as file:
+        least, most = map(int, re.search(r"kScaledArcMin = (-?\d+), kScaledArcMax = (-?\d+)", file.read()).groups())
+    assert -LAG + 2 * (least - 1) >= -1022
+    assert 4 * (2 * (most + 1) + SLOPE) < 1023 and 8 * (most + 1 + SLOPE) < 1023
