@@ -102,6 +102,7 @@ def _draw_seed(dropout, seed):
 def joint_dropout_mask(B, T, U, H, dropout, seed, device):
     """The keep mask [B,T,U,H] (bool) the kernels derive from (seed, cell, hidden unit), for tests."""
     mask = torch.empty(B, T, U, H, dtype=torch.uint8, device=device)
+    device = mask.device  # (whatever torch takes for a device: a name, a number)
     with _on(device):
         status = _native.lib().mi_joint_dropout_mask(_ptr(mask), float(dropout), int(seed), B, T, U, H, _stream(device))
     _native.check_status(status, "joint_dropout_mask")

@@ -169,6 +169,11 @@ def test_dropout_mask_is_a_function_of_the_seed_and_keeps_the_right_share(p):
     assert joint_dropout_mask(2, 3, 4, 512, 0.0, 7, DEV).all()
 
 
+@pytest.mark.parametrize("device", [0, "cuda", torch.device("cuda"), torch.device("cuda", 0)])
+def test_dropout_mask_takes_a_device_as_torch_does(device):
+    assert torch.equal(joint_dropout_mask(2, 3, 4, 512, 0.5, 7, device), joint_dropout_mask(2, 3, 4, 512, 0.5, 7, DEV))
+
+
 @pytest.mark.parametrize("H,p", [(640, 0.2), (512, 0.5)])
 def test_dropout_parity_with_the_exported_mask(H, p):
     B, T, U, V = 3, 9, 6, 130
