@@ -4,7 +4,7 @@ many utterances (a wave takes 64 at a time), and the checks of the loss modules 
 import pytest
 import torch
 
-from speech_amd import MultiblankRNNTLossNumba, RNNTLossNumba, TDTLossNumba
+from speech_amd import MultiblankRNNTLossNumba, RNNTLossNumba, TDTLossNumba, _native
 from speech_amd.rnnt_loss import rnnt
 
 from gpu_utils import DEV
@@ -12,7 +12,14 @@ from gpu_utils import DEV
 pytestmark = pytest.mark.gpu
 
 # V and dtype of a row: by tile, by wave, by workgroup, streamed (more than 8192 vectors of 16 bytes)
-ROWS = [(29, torch.float32), (1025, torch.float32), (1025, torch.bfloat16), (2100, torch.float16), (40000, torch.float32)]
+ROWS = [(29, torch.float32), (1025, torch.float32), (1025, torch.bfloat16), (2100, torch.float16), (4097, torch.float32), (16385, torch.bfloat16),
+        (40000, torch.float32)]  # fmt: skip
+
+
+def test_the_rows_reach_every_kernel_of_pass_1():
+    code = {torch.float32: _native.DTYPE_F32, torch.bfloat16: _native.DTYPE_BF16, torch.float16: _native.DTYPE_F16}
+    kernels = {_native.describe_plan(code[dtype], 3, 3, 2, V)["denominators"].split("<")[0] for V, dtype in ROWS}
+    assert kernels == {"denom_tile_kernel", "denom_rows_kernel", "denom_block_kernel", "denom_gather_kernel"}
 
 
 @pytest.mark.parametrize("V,dtype", ROWS)
