@@ -74,10 +74,12 @@ def test_multiblank_forward_backward_in_a_graph():
     eager_and_graph("multiblank", 3, 17, 6, 40, {"big": [2, 4]}, 3)
 
 
-def test_fused_joint_forward_and_backward_replay_from_a_graph():
+@pytest.mark.parametrize("sums", ["two passes", "one pass"])
+def test_fused_joint_forward_and_backward_replay_from_a_graph(sums):
     """The fused joint's step reads nothing back from the device (its row buffers are sized by a bound the host
     knows, the tiles in use are counted and consumed on the device), so the C-level forward, backward and reduction
-    can be captured and replayed on new inputs -- with other lengths, i.e. another number of tiles in use."""
+    (a sum a pass, or mi_joint_gradient_sums with every sum in its gradient's dtype) can be captured and replayed on new
+    inputs -- with other lengths, i.e. another number of tiles in use."""
     import ctypes
 
     from speech_amd import _native
@@ -102,8 +104,10 @@ def test_fused_joint_forward_and_backward_replay_from_a_graph():
     d_hidden = torch.empty(tiles * 128, H, dtype=torch.bfloat16, device=DEV)
     scale = torch.ones(B, device=DEV)
 
+    chunks = (T + 15) // 16
+
     def run(out):
-        costs, dw, db, df, dg = out
+        costs, dw, db, df, dg, dg_part, d_weight, d_bias = out
         stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
         args = (B, T, U, H, V, V - 1)
         st = lib.mi_joint_rnnt_forward(f.data_ptr(), g.data_ptr(), W.data_ptr(), bias.data_ptr(), _native.DTYPE_F32,
@@ -115,14 +119,22 @@ def test_fused_joint_forward_and_backward_replay_from_a_graph():
                                         d_hidden.data_ptr(), dw.data_ptr(), db.data_ptr(), slices, tiles, scale.data_ptr(),
                                         1, 1.0, *args, 0.01, 0.0, ws.data_ptr(), ws.numel(), stream)  # fmt: skip
         assert st == _native.SUCCESS
-        st = lib.mi_joint_reduce_hidden(d_hidden.data_ptr(), f.data_ptr(), g.data_ptr(), al.data_ptr(), ll.data_ptr(),
-                                        df.data_ptr(), dg.data_ptr(), None, 0, tiles, 0.0, 0, 0, B, T, U, H, V, 0, 0,
-                                        ws.data_ptr(), ws.numel(), stream)  # fmt: skip
+        if sums == "one pass":
+            st = lib.mi_joint_gradient_sums(d_hidden.data_ptr(), f.data_ptr(), g.data_ptr(), al.data_ptr(), ll.data_ptr(),
+                                            df.data_ptr(), _native.DTYPE_F32, dg_part.data_ptr(), chunks, dg.data_ptr(),
+                                            _native.DTYPE_F32, dw.data_ptr(), db.data_ptr(), slices, d_weight.data_ptr(),
+                                            _native.DTYPE_BF16, d_bias.data_ptr(), _native.DTYPE_F16, tiles, 0.0, 0, 0,
+                                            B, T, U, H, V, 0, 0, ws.data_ptr(), ws.numel(), stream)  # fmt: skip
+        else:
+            st = lib.mi_joint_reduce_hidden(d_hidden.data_ptr(), f.data_ptr(), g.data_ptr(), al.data_ptr(), ll.data_ptr(),
+                                            df.data_ptr(), dg.data_ptr(), None, 0, tiles, 0.0, 0, 0, B, T, U, H, V, 0, 0,
+                                            ws.data_ptr(), ws.numel(), stream)  # fmt: skip
         assert st == _native.SUCCESS
 
     def outputs():
         return (torch.empty(B, device=DEV), torch.empty(slices, NP, H, device=DEV), torch.empty(slices, NP, device=DEV),
-                torch.empty(B, T, H, device=DEV), torch.empty(B, U, H, device=DEV))
+                torch.empty(B, T, H, device=DEV), torch.empty(B, U, H, device=DEV), torch.empty(chunks, B, U, H, device=DEV),
+                torch.zeros(V, H, dtype=torch.bfloat16, device=DEV), torch.zeros(V, dtype=torch.float16, device=DEV))  # fmt: skip
 
     eager, captured = outputs(), outputs()
     f.copy_(torch.tensor(rng.randn(B, T, H), dtype=torch.bfloat16))
@@ -145,5 +157,9 @@ def test_fused_joint_forward_and_backward_replay_from_a_graph():
         torch.cuda.synchronize()
         run(eager)  # the program's own eager work between replays
         torch.cuda.synchronize()
-        for name, x, y in zip(("costs", "dw", "db", "df", "dg"), captured, eager):
-            assert torch.equal(x, y), (name, replay)
+        for name, x, y in zip(("costs", "dw", "db", "df", "dg", "dg parts", "d weight", "d bias"), captured, eager):
+            if sums == "one pass" or name in ("costs", "dw", "db", "df", "dg"):
+                assert torch.equal(x, y), (name, replay)
+        if sums == "one pass":  # (each of them was written in the replay: they are sums of what is not -3)
+            assert torch.allclose(captured[6].float(), captured[1].sum(0)[:V], rtol=2.0**-7, atol=1e-4)
+            assert torch.allclose(captured[4], captured[5].sum(0), rtol=1e-5, atol=1e-5)
