@@ -1,6 +1,6 @@
 """TDT and multi-blank lattices on probabilities with shared exponents (mi_scaled.inc), against the oracle: the edges of their
 groups of 64 columns, batches of diagonals and longest durations, and the inputs that send them to the same recursion on
-logarithms (arcs below exp(-60), columns far apart, totals near the sentinels, values that are not numbers)."""
+logarithms (arcs below exp(-693), cells far below their columns, columns far apart, totals near the sentinels, values that are not numbers)."""
 
 import numpy as np
 import pytest
@@ -78,10 +78,23 @@ def test_many_diagonals(kind, steps):
 @pytest.mark.parametrize("kind,steps,scale", [("tdt", [0, 1, 2, 3, 4], 30.0), ("tdt", [0, 1, 2, 6], 25.0),
                                               ("multiblank", [2, 4, 8], 30.0), ("multiblank", [2], 300.0)])  # fmt: skip
 def test_arcs_below_the_range(kind, steps, scale):
-    """Log-probs of -60 and far beyond: the recursion on logarithms decides.  (TDT with totals above the sentinels' -10000:
+    """Log-probs of -60 and far beyond, most of them: the recursion on logarithms decides most.  (TDT with totals above the sentinels' -10000:
     below, the oracle's own posteriors overflow.  Rounding: log-probs of 1000, 2^-24 of each.)"""
     acts, labels, act_lens, label_lens = draw(11, kind, 4, 21, 70, steps)
     check(kind, acts * scale, labels, act_lens, label_lens, steps, cost_rtol=2e-6, grad_atol=60 * 1000 * 2.0**-24)
+
+
+@gpu
+@pytest.mark.parametrize("value", [-70.0, -150.0, -600.0, -686.0, -700.0, -5000.0])
+@pytest.mark.parametrize("kind,steps", [("tdt", [0, 1, 2, 3, 4]), ("tdt", [0, 1, 8]), ("multiblank", [2, 4, 8]), ("multiblank", [2])])
+@pytest.mark.parametrize("T,U", [(40, 1), (30, 9), (21, 70), (12, 140)])
+def test_few_dear_arcs_among_ordinary_ones(kind, steps, value, T, U):
+    """Log-probs of `value` in one cell of a hundred, on both sides of the range's lower end.  What passes through such an arc carries
+    its rounding, 2^-24 of 690 (beyond: of the gradient's share of next to nothing), and without labels a path may need three."""
+    acts, labels, act_lens, label_lens = draw(13, kind, 3, T, U, steps)
+    rng = np.random.RandomState(U)
+    acts[rng.rand(*acts.shape) < 0.01] = value
+    check(kind, acts, labels, act_lens, label_lens, steps, cost_rtol=2e-6, grad_atol=3 * 700 * 2.0**-24)
 
 
 @gpu
@@ -120,9 +133,9 @@ def test_plan_lines():
     """Which lattice a shape gets: 256 columns, 192 with a longest duration above 4, durations up to 8."""
     for U, longest, scaled in [(121, 4, True), (256, 4, True), (257, 4, False), (192, 8, True), (193, 8, False), (64, 9, False)]:
         tdt = _native.describe_plan(0, 4, 100, U, 65, D=5, max_duration=longest)["lattice"]
-        assert (tdt == "tdt_lattice_pair_kernel<D=5>") == scaled, (U, longest, tdt)
+        assert tdt.startswith("tdt_lattice_pair_kernel<") == scaled, (U, longest, tdt)
         mb = _native.describe_plan(0, 4, 100, U, 68, max_duration=longest, num_big_blanks=3)["lattice"]
-        assert (mb == "multiblank_lattice_kernel<NBC=4>") == scaled, (U, longest, mb)
+        assert mb.startswith("multiblank_lattice_kernel<") == scaled, (U, longest, mb)
 
 
 @gpu

@@ -96,9 +96,10 @@ def recursion(tdt, longest, beta, factors, diagonals, steps, batch):
     return values, exponents
 
 
-def guard(tdt, durations, longest, values, exponents, end, T, batch):
+def guard(tdt, durations, longest, values, exponents, last, T, batch):
     """Whether a lattice runs again on logarithms, as the helpers find out batch by batch."""
     n, total, columns = values.shape
+    end = values[:, last, -1]
     i, pos = np.arange(total)[:, None], np.arange(columns)[None]
     valid = (i >= pos) & (i - pos < T)
     mass = high_word(values) > 0
@@ -110,6 +111,9 @@ def guard(tdt, durations, longest, values, exponents, end, T, batch):
     for q in range(low.shape[1]):
         for w in range(min(q, (batch - 1 + longest) // batch) + 1):
             bad |= ((low[:, q - w] < high[:, q] - LAG) | (low[:, q] < high[:, q - w] - LAG)).any(1)
+    q = last // batch  # (the total: alpha's lies behind the last cell)
+    for w in range(min(q, (batch - 1 + longest) // batch) + 1):
+        bad |= np.frexp(end)[1] + exponents[:, last, -1] < high[:, q - w, -1] - LAG
     return bad
 
 
@@ -171,7 +175,7 @@ def compare(tdt, durations, blank, label, ways, batch=None):
             factors[..., d + (2 if tdt else 0)] = np.where(valid[..., 0], np.exp(ways[:, t, u, k]), 1.0 if tdt else 0.0)
         values, exponents = recursion(tdt, longest, beta, factors, diagonals, steps, batch)
         end = values[:, steps - 1, U - 1]
-        verdicts.append(guard(tdt, durations, longest, values, exponents, end, T, batch))
+        verdicts.append(guard(tdt, durations, longest, values, exponents, steps - 1, T, batch))
         t, u = np.meshgrid(np.arange(T), np.arange(U), indexing="ij")
         at = (diagonals - 1 - t - u, U - 1 - u) if beta else (t + u, u)
         mantissa, exponent = np.frexp(values[:, at[0], at[1]])
@@ -188,7 +192,7 @@ def compare(tdt, durations, blank, label, ways, batch=None):
 
 
 # What a pattern varies over (lattice only, cells, columns, frames, quarters of the lattice), each arc either dear or cheap
-def arcs(rng, pattern, n, T, U, dear=-59.9):
+def arcs(rng, pattern, n, T, U, dear):
     t, u = np.arange(T)[None, :, None], np.arange(U)[None, None]
     if pattern == "lattice":
         x = np.where(rng.rand(n, 1, 1) < 0.6, dear * rng.rand(n, 1, 1), -0.1)
@@ -209,16 +213,33 @@ BLANK_SETS = [[1, 2], [1, 4], [1, 2, 4, 8], [1, 8], [1, 3, 5, 7]]  # (the standa
 
 
 @pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("dear", [-59.9, -170.0, -690.0])
 @pytest.mark.parametrize("pattern", ["lattice", "cells", "columns", "frames", "quarters"])
 @pytest.mark.parametrize("tdt,durations", [(True, d) for d in TDT_SETS] + [(False, d) for d in BLANK_SETS])
-def test_what_the_guard_passes_is_right(pattern, tdt, durations):
-    """A value's relative error is some 2^-53 a step, and the logarithms' own rounding up to (T + U) * 120 * 2^-53 = 2e-12."""
+def test_what_the_guard_passes_is_right(pattern, tdt, durations, dear):
+    """A value's relative error is some 2^-53 a step, and the logarithms' own rounding up to (T + U) * 1400 * 2^-53 = 2e-11."""
     rng = np.random.RandomState(len(pattern) + 100 * sum(durations) + tdt)
     for T, U in [(25, 1), (9, 2), (17, 5), (30, 9), (8, 40), (5, 70)]:
-        blank, label = arcs(rng, pattern, 10, T, U), arcs(rng, pattern, 10, T, U)
-        ways = np.stack([arcs(rng, pattern, 10, T, U) for _ in durations], -1)
+        blank, label = arcs(rng, pattern, 10, T, U, dear), arcs(rng, pattern, 10, T, U, dear)
+        ways = np.stack([arcs(rng, pattern, 10, T, U, dear) for _ in durations], -1)
         verdicts, errors = compare(tdt, durations, blank, label, ways)
         assert not (errors[~verdicts] > 1e-10).any(), (T, U, errors[~verdicts].max())
+
+
+@pytest.mark.filterwarnings("ignore::RuntimeWarning")
+@pytest.mark.parametrize("tdt,durations", [(True, d) for d in TDT_SETS] + [(False, d) for d in BLANK_SETS])
+def test_few_dear_arcs_among_ordinary_ones(tdt, durations):
+    """Log-probs of down to -690 in one cell of a hundred: right, and without the recursion on logarithms where another path leads to
+    every cell."""
+    rng = np.random.RandomState(sum(durations))
+
+    def draw(T, U):
+        return np.where(rng.rand(8, T, U) < 0.01, -690 * rng.rand(8, T, U), -3 * rng.rand(8, T, U))
+
+    for T, U in [(40, 1), (30, 6), (75, 70)]:
+        verdicts, errors = compare(tdt, durations, draw(T, U), draw(T, U), np.stack([draw(T, U) for _ in durations], -1))
+        assert not (errors[~verdicts] > 1e-10).any(), (T, U, errors[~verdicts].max())
+        assert U == 1 or not verdicts.all(), (T, U)
 
 
 @pytest.mark.filterwarnings("ignore::RuntimeWarning")
@@ -227,9 +248,9 @@ def test_what_the_guard_passes_is_right(pattern, tdt, durations):
 def test_every_arc_at_one_level(tdt, durations, U):
     """Runs of short steps beside long ones, and columns that cost 174 bits each.  (The random patterns rarely need the distances
     that the guard watches, cells without mass tell nearly all; of these, TDT with [0, 1, 8] and 70 columns with any set do.)"""
-    levels = np.linspace(-59.9, -30.0, 8)[:, None, None]
+    levels = np.array([-690.0, -400.0, -250.0, -150.0, -100.0, -80.0, -59.9, -55.0, -50.0, -45.0, -40.0, -30.0])[:, None, None]
     for T in range(2, 34, 1 if U < 5 else 3) if U < 70 else (3, 4, 5, 6):
-        dear = np.broadcast_to(levels, (8, T, U))
+        dear = np.broadcast_to(levels, (len(levels), T, U))
         verdicts, errors = compare(tdt, durations, dear, dear, np.stack([dear] * len(durations), -1))
         assert not (errors[~verdicts] > 1e-10).any(), (T, errors[~verdicts].max())
 
@@ -259,9 +280,11 @@ def test_ordinary_lattices_pass(tdt, durations, spread):
 
 
 def test_the_bounds_fit_a_double():
-    """A cell LAG bits down pushes through two arcs at the lower bound, with the rounding of an exponent each: normal still.  Upwards,
-    four steps (TDT: two arcs each) or eight of the largest factors and slopes stay finite."""
+    """What is lost, below 2^-1022 of a column's exponent, of the one below (SLOPE higher) and a factor short of arriving, or in the own
+    column and two short, is less than 2^-80 of a cell LAG bits down.  An arc at the lower bound is a normal number.  Upwards, four
+    steps (TDT: two arcs each) or eight of the largest factors and slopes stay finite."""
     with open(SOURCE) as file:
         least, most = map(int, re.search(r"kScaledArcMin = (-?\d+), kScaledArcMax = (-?\d+)", file.read()).groups())
-    assert -LAG + 2 * (least - 1) >= -1022
+    assert 1022 - LAG - SLOPE - (most + 1) >= 80 and 1022 - LAG - 2 * (most + 1) >= 80
+    assert least - 1 > -1022
     assert 4 * (2 * (most + 1) + SLOPE) < 1023 and 8 * (most + 1 + SLOPE) < 1023
