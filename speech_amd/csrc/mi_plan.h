@@ -193,7 +193,7 @@ struct ScaledPlan {
 // Batches of 8 diagonals and four helpers a group, as far as LDS holds them and for one or two groups; beyond, batches of 4,
 // and two helpers: four groups then have the twelve waves that a compute unit gives enough registers.
 // longest == 0: longer durations, more than 256 columns (192 with a longest duration above 4), more LDS than there is.
-inline ScaledPlan scaled_plan(bool tdt, int longest, int U) {
+constexpr ScaledPlan scaled_plan(bool tdt, int longest, int U) {
   const int groups = (U + 63) / 64, maxd = longest <= 4 ? 4 : 8, factors = scaled_factors(tdt, maxd);
   ScaledPlan p{0, 0, 0, 0, 0};
   if (longest > 8 || groups > kScaledMaxGroups) return p;
@@ -204,6 +204,15 @@ inline ScaledPlan scaled_plan(bool tdt, int longest, int U) {
     return ScaledPlan{maxd, steps, helpers, 64 * groups * (1 + helpers), lds};
   }
   return p;
+}
+// the largest workgroup that any plan launches an instantiation with
+constexpr int scaled_threads(bool tdt, int longest, int steps, int helpers) {
+  int most = 0;
+  for (int groups = 1; groups <= kScaledMaxGroups; ++groups) {
+    const ScaledPlan p = scaled_plan(tdt, longest, 64 * groups);
+    if (p.longest == longest && p.steps == steps && p.helpers == helpers && p.threads > most) most = p.threads;
+  }
+  return most;
 }
 // offsets into an utterance's records are 32-bit (and run up to 256 diagonals past its end)
 inline bool scaled_offsets_fit(const Layout& L) { return (L.ND + 256LL) * L.Us * L.A * 4 < (1LL << 31); }

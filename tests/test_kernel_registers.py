@@ -1,6 +1,7 @@
-"""What the compiler made of the joint forward: its operands (up to 328 registers a lane) have to stay in registers.  An
-instantiation whose arrays went to scratch gives the right results, only slower, so no other test sees it.  Read from the
-resource records of the library that was built here; nothing is launched."""
+"""What the compiler made of the joint forward, whose operands (up to 328 registers a lane) have to stay in registers, and of the
+lattices on probabilities, whose helper waves count their loads and stores in flight.  An instantiation whose arrays went to scratch gives
+the right results, only slower, so no other test sees it.  Read from the resource records of the library that was built here;
+nothing is launched."""
 
 import os
 import re
@@ -56,4 +57,19 @@ def test_joint_forward_uses_no_scratch(kernels, H):
         if m and int(m[1]) == H:
             found[m.groups()[1:]] = kernel[".private_segment_fixed_size"]
     assert len(found) == 3 * 2 * 2 * 2  # losses, ReLU or smooth, with and without the backward's operands, groups of cells
+    assert not any(found.values()), {k: v for k, v in found.items() if v}
+
+
+# MAXD, diagonals a batch, helper waves, and the largest workgroup launched: up to two groups of 64 columns, three or four, ...
+LATTICES = [(4, 8, 4, 640), (4, 4, 2, 768), (8, 8, 4, 320), (8, 4, 4, 640), (8, 4, 2, 576)]
+
+
+@pytest.mark.parametrize("kernel", ["tdt_lattice_pair_kernel", "multiblank_lattice_kernel"])
+def test_lattices_on_probabilities_use_no_scratch(kernels, kernel):
+    found = {}
+    for name, record in kernels.items():
+        m = re.search(rf"{kernel}ILi(\d)ELi(\d)ELi(\d)EE", name)
+        if m:
+            found[tuple(map(int, m.groups())) + (record[".max_flat_workgroup_size"],)] = record[".private_segment_fixed_size"]
+    assert sorted(found) == sorted(LATTICES)
     assert not any(found.values()), {k: v for k, v in found.items() if v}
