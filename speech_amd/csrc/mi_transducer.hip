@@ -596,10 +596,11 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   else snprintf(denom, sizeof denom, "denom_gather_kernel<%s>", dt);
   const bool tdt = D > 0 && !use_plain_rnnt;
   const bool mb = num_big_blanks > 0;
+  const ScaledPlan sp = (tdt || mb) && scaled_offsets_fit(c.L) ? scaled_plan(tdt, max_duration, U) : ScaledPlan{0, 0, 0, 0, 0};
   if (mb) {
     const int nbc = num_big_blanks <= 1 ? 1 : (num_big_blanks <= 2 ? 2 : (num_big_blanks <= 4 ? 4 : 8));
     const size_t lds = (size_t)(max_duration + 1) * (2 + nbc) * c.L.Us * sizeof(double);
-    if (scaled_plan(false, max_duration, U).longest) snprintf(lattice, sizeof lattice, "multiblank_lattice_kernel<NBC=%d>", nbc);
+    if (sp.longest) snprintf(lattice, sizeof lattice, "multiblank_lattice_kernel<MAXD=%d, P=%d, H=%d>", sp.longest, sp.steps, sp.helpers);
     else if (lds > 160 * 1024) snprintf(lattice, sizeof lattice, "multiblank_lattice_pull_kernel");
     else snprintf(lattice, sizeof lattice, "multiblank_lattice_ring_kernel<NBC=%d>", nbc);
   } else if (D == 0 || use_plain_rnnt) {
@@ -607,8 +608,8 @@ int mi_transducer_describe_plan(int act_dtype, int B, int T, int U, int V, int D
   } else {
     const int R = max_duration + 2;
     const size_t lds_block = (size_t)R * 2 * D * c.L.Us * sizeof(double);
-    if (scaled_plan(true, max_duration, U).longest) snprintf(lattice, sizeof lattice, "tdt_lattice_pair_kernel<D=%d>", D);
-    else if (D <= 8 && c.L.Us <= 256 && lds_block <= 160 * 1024) snprintf(lattice, sizeof lattice, "tdt_lattice_ring_kernel<D=%d>", D);
+    if (sp.longest) snprintf(lattice, sizeof lattice, "tdt_lattice_pair_kernel<MAXD=%d, P=%d, H=%d>", sp.longest, sp.steps, sp.helpers);
+    else if (D >= 2 && D <= 8 && c.L.Us <= 256 && lds_block <= 160 * 1024) snprintf(lattice, sizeof lattice, "tdt_lattice_ring_kernel<D=%d>", D);
     else snprintf(lattice, sizeof lattice, "tdt_lattice_kernel<K=%d>", c.L.K);
   }
   // a gradient buffer at the 16-byte phase of the logits is assumed (what every allocator returns)

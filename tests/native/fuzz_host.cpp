@@ -74,6 +74,21 @@ static void fuzz_tiles(const PlanShape& s) {
   }
 }
 
+// Lattices on probabilities: a plan has to be one of the launchers' instantiations, hold the lattice and fit a compute unit.
+static void fuzz_scaled(const Layout& L, int U, const ScaledPlan& p, bool tdt, int longest, bool distinct) {
+  const int groups = (U + 63) / 64, factors = scaled_factors(tdt, longest <= 4 ? 4 : 8);
+  const bool fits = (L.ND + 256LL) * L.Us * L.A * 4 < (1LL << 31) && groups * scaled_group_bytes(factors, 4) + 16 <= 160 * 1024;
+  EXPECT((p.longest != 0) == (distinct && fits && longest <= 8 && U <= 256), "longest %d U %d ND %d tdt %d", longest, U, L.ND, tdt);
+  if (!p.longest) return;
+  static const int forms[][3] = {{4, 8, 4}, {4, 4, 2}, {8, 8, 4}, {8, 4, 4}, {8, 4, 2}};  // MAXD, P, H
+  bool known = false;
+  for (const auto& f : forms) known |= p.longest == f[0] && p.steps == f[1] && p.helpers == f[2];
+  EXPECT(known && p.longest >= longest, "MAXD %d P %d H %d for %d", p.longest, p.steps, p.helpers, longest);
+  EXPECT(p.threads == 64 * groups * (1 + p.helpers) && p.threads <= scaled_threads(tdt, p.longest, p.steps, p.helpers), "threads %d U %d", p.threads, U);
+  EXPECT(p.lds <= 160 * 1024 && p.lds >= groups * scaled_group_bytes(factors, p.steps) + 3 * sizeof(int), "lds %zu U %d", p.lds, U);
+  EXPECT(factors >= (tdt ? 3 : 1) + p.longest && factors % 2 == 0, "factors %d", factors);
+}
+
 static void fuzz_plan(std::mt19937& rng, int iterations) {
   auto uni = [&](int lo, int hi) { return std::uniform_int_distribution<int>(lo, hi)(rng); };
   for (int it = 0; it < iterations; ++it) {
@@ -135,6 +150,18 @@ static void fuzz_plan(std::mt19937& rng, int iterations) {
     const int ms = make_mb_params(nbb, bd, 0.f, &mp);
     EXPECT((ms == MI_TRANSDUCER_SUCCESS) == bd_ok, "big blanks n %d", nbb);
     if (ms == MI_TRANSDUCER_SUCCESS) EXPECT(mp.R == longest + 1, "ring depth");
+    Layout SL;
+    const int long_T = uni(0, 3) ? uni(1, 2000) : uni(1, 524280), narrow_U = uni(1, 300);
+    if (st == MI_TRANSDUCER_SUCCESS && make_layout(1, long_T, narrow_U, nd, &SL))
+      fuzz_scaled(SL, narrow_U, scaled_plan(SL, tp, narrow_U), true, dur[nd - 1], true);
+    if (ms == MI_TRANSDUCER_SUCCESS) {
+      for (int i = 0; i < nbb && uni(0, 3); ++i) bd[i] = uni(1, 10);  // (mostly those in use)
+      make_mb_params(nbb, bd, 0.f, &mp);
+      bool distinct = nbb > 0;
+      for (int i = 0; i < nbb; ++i)
+        for (int j = 0; j <= i; ++j) distinct = distinct && (i == j ? bd[i] >= 2 : bd[i] != bd[j]);
+      if (make_layout(1, long_T, narrow_U, nbb, &SL)) fuzz_scaled(SL, narrow_U, scaled_plan(SL, mp, narrow_U), false, mp.R - 1, distinct);
+    }
     // kernel shapes: whatever is chosen must cover the row and fit a workgroup
     PlanShape s;
     s.dt = uni(0, 2); s.B = uni(1, 64); s.T = uni(1, 800); s.U = uni(1, uni(0, 1) ? 1024 : 40);

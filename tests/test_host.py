@@ -73,12 +73,12 @@ def test_kernel_plan_of_the_documented_shapes(built_lib):
     assert p["denominators"] == "denom_gather_kernel<f32>" and p["gradient"] == "grad_stream_kernel<f32>"
     assert p["cells"] == "rnnt_cell_kernel"
     p = plan(F32, 16, 375, 121, 1025, D=5, max_duration=4)  # TDT: coefficients come from the cell kernel
-    assert p["lattice"] == "tdt_lattice_pair_kernel<D=5>" and p["cells"] == "tdt_cell_kernel"
+    assert p["lattice"] == "tdt_lattice_pair_kernel<MAXD=4, P=8, H=4>" and p["cells"] == "tdt_cell_kernel"
     assert p["gradient"] == "grad_block_kernel<f32, RT=128, NVT=2, coef>"
     p = plan(F32, 16, 375, 121, 1025, D=5, max_duration=4, use_plain_rnnt=True)
     assert p["lattice"] == "rnnt_lattice_kernel<K=2>" and p["cells"] == "-"
     p = plan(F32, 16, 375, 121, 1028, num_big_blanks=3)  # multi-blank: three big blanks inside V
-    assert p["lattice"] == "multiblank_lattice_kernel<NBC=4>" and p["cells"] == "multiblank_cell_kernel"
+    assert p["lattice"] == "multiblank_lattice_kernel<MAXD=4, P=8, H=4>" and p["cells"] == "multiblank_cell_kernel"
     # 257 whole vectors, one past a power of two: 5 vectors per lane in pass 1, a third (nearly empty) vector per
     # thread in the gradient pass rather than twice the threads
     assert p["denominators"] == "denom_rows_kernel<f32, R=5, RPW=1>"
@@ -109,6 +109,25 @@ def test_kernel_plan_of_rows_about_64_vectors(built_lib):
                 by_rows = vec == 8 and (40 if D else 56) < vectors <= 64
                 assert gradient == ("grad_block_kernel" if vectors > 64 else "grad_rows_kernel" if by_rows else "grad_tile_kernel"), V
                 assert p["cells"] == ("tdt_cell_kernel" if D else "rnnt_cell_kernel" if vectors <= 64 else "-")
+
+
+def test_kernel_plan_of_lattices_on_probabilities(built_lib):
+    """The longest duration an instantiation holds, diagonals a batch and helper waves, by columns; lattices whose records take 2^31
+    bytes are left to the kernels on logarithms (one duration: to a wave a lattice, which any number of them can have)."""
+    for longest, lines in [(4, {1: (4, 8, 4), 64: (4, 8, 4), 128: (4, 8, 4), 129: (4, 4, 2), 256: (4, 4, 2), 257: None}),
+                           (8, {1: (8, 8, 4), 64: (8, 8, 4), 65: (8, 4, 4), 128: (8, 4, 4), 129: (8, 4, 2), 192: (8, 4, 2), 193: None}),
+                           (9, {1: None})]:  # fmt: skip
+        for U, shape in lines.items():
+            tdt = _native.describe_plan(0, 4, 100, U, 65, D=5, max_duration=longest)["lattice"]
+            mb = _native.describe_plan(0, 4, 100, U, 68, max_duration=longest, num_big_blanks=3)["lattice"]
+            if shape is None:
+                assert "pair" not in tdt and not mb.startswith("multiblank_lattice_kernel"), (U, longest, tdt, mb)
+            else:
+                form = "<MAXD={}, P={}, H={}>".format(*shape)
+                assert (tdt, mb) == ("tdt_lattice_pair_kernel" + form, "multiblank_lattice_kernel" + form), (U, longest)
+    for D, name in [(1, "tdt_lattice_kernel<K=4>"), (2, "tdt_lattice_ring_kernel<D=2>")]:
+        assert _native.describe_plan(0, 1, 524000, 256, 9, D=D, max_duration=1)["lattice"] == name
+    assert _native.describe_plan(0, 1, 524000, 256, 9, max_duration=2, num_big_blanks=1)["lattice"] == "multiblank_lattice_ring_kernel<NBC=1>"
 
 
 def test_constructor_attributes_match_the_reference_conventions():
