@@ -288,3 +288,30 @@ def test_the_bounds_fit_a_double():
     assert 1022 - LAG - SLOPE - (most + 1) >= 80 and 1022 - LAG - 2 * (most + 1) >= 80
     assert least - 1 > -1022
     assert 4 * (2 * (most + 1) + SLOPE) < 1023 and 8 * (most + 1 + SLOPE) < 1023
+
+
+def test_exponents_of_the_factors_from_the_bits_of_a_float():
+    """n = rint(x log2(e)) is formed as 1.5 2^23 + n in one float32 multiply-add.  Within the guard's range its bits less those of
+    1.5 2^23 are n, |x log2(e) - n| <= 1/2 (and what float32's log2(e) and the rounding of 2^f leave) and 2^n fits a double's
+    exponent; outside it, infinities and NaN included, the bits lie outside the guard's bounds, as signed integers."""
+    log2e, base = np.float32(1.44269502), np.float32(12582912.0)
+    x = np.concatenate([np.linspace(-693.2, 20.2, 200001), -np.logspace(-30, 2.8, 4001), [0.0, -0.0]]).astype(np.float32)
+    low, high = 0x4B400000 - 1000, 0x4B400000 + 29
+
+    def bits(x):
+        with np.errstate(over="ignore", invalid="ignore"):  # (the product of two float32 is exact in float64)
+            return (x.astype(np.float64) * np.float64(log2e) + np.float64(base)).astype(np.float32).view(np.int32)
+
+    n = bits(x).astype(np.int64) - 0x4B400000
+    exact = x.astype(np.float64) * np.log2(np.e)
+    assert np.abs(exact - n).max() <= 0.5 + 1000 * 2.0**-24
+    mantissa = np.exp2(exact - n)
+    factor = ((mantissa.view(np.int64) + (n << 52)).view(np.float64))
+    np.testing.assert_allclose(factor, np.exp(x.astype(np.float64)), rtol=1e-12)
+    inside = (bits(x) >= low) & (bits(x) <= high)
+    assert np.array_equal(inside, (np.rint(exact) >= -1000) & (np.rint(exact) <= 29))
+    outside = np.array([-693.9, -700.0, -1.0e4, -2.0e6, -2.9e6, -4.0e6, -5.9e6, -1.0e7, -1.0e10, -3.4e38, -np.inf,
+                        20.5, 700.0, 2.0e6, 1.0e7, 3.4e38, np.inf, np.nan], dtype=np.float32)  # fmt: skip
+    b = bits(outside)
+    assert not ((b >= low) & (b <= high)).any()
+    assert (b[:11] < low).all() and (b[11:] > high).all()
