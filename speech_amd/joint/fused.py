@@ -292,11 +292,12 @@ class JointRNNTLoss(torch.autograd.Function):
         want_f, want_g = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         # Both of d f and d g wanted (the usual case): one pass over d_hidden forms d f and, per run of frames, a share of d g
         # (runs of a length that U alone decides: the sums then do not depend on how a batch is split into sub-batches).
-        # A workgroup walks its run frame by frame, a barrier each: shorter runs give more workgroups, longer ones
-        # fewer partial sums to add.  Runs of 16 frames against 32, us: the reduction at B=4, T=190, U=49, H=640
-        # 27 / 48; a step at B=16, T=375, H=640, V=257: U=33 472 / 469, U=64 710 / 703, U=121 1139 / 1138.  Few
-        # utterances gain from 16 at larger U too (B=8, T=250, H=256: U=96 270 / 289, U=121 306 / 331), but their
-        # number must not decide.
+        # A workgroup walks its run frame by frame, a barrier every four: shorter runs give more workgroups, longer ones
+        # fewer partial sums to add.  Runs of 16 frames / 32, us: a step, and the reduction with the sums behind it, at
+        # B=16, T=375, H=640, V=257: U=33 443 / 449, 83 / 89; U=64 703 / 710, 109 / 117; U=65 707 / 697, 124 / 115; U=121
+        # 1183 / 1170, 178 / 164; U=200 1854 / 1823, 282 / 255; at B=4, T=190, U=49, V=1025 253 / 263, 31 / 41.  Few
+        # utterances gain from 16 at larger U too (B=8, T=250, H=256: U=96 272 / 280, U=121 323 / 337), but their number
+        # must not decide.
         run = 16 if U <= 64 else 32
         one_pass = want_f and want_g and U <= 256
         chunks = (T + run - 1) // run if one_pass else 0
